@@ -25,19 +25,37 @@ namespace fufft {
 
 constexpr int cpb_for(int T) { return T >= 128 ? 1 : 256 / T; }
 
-// Transform groups one workgroup of the single-launch conv runs in turn.  At
+// Transforms one workgroup of the single-launch conv runs in turn.  At
 // N = 16384 the transform fills a CU's LDS, one workgroup per CU, and each
 // new workgroup starts some 1200 cycles after the last left; eight in a row
-// measured 225.3 -> 232.8 and 225.6 -> 230.0 Gpt/s (two boxes, each against
-// one per workgroup), the digit-order filter 218.8 -> 223.4.  Elsewhere the
-// other resident workgroups hide the start, and the loop cost 3-11%
-// (N = 512 .. 8192, 2 to 8 in a row).
+// measured 225.3 -> 232.8 and 225.6 -> 230.0 Gpt/s (two boxes, 2^27 points,
+// each against one per workgroup), the digit-order filter 218.8 -> 223.4.
+// Elsewhere the other resident workgroups hide the start, and the loop cost
+// 3-11% (N = 512 .. 8192, 2 to 8 in a row).
 // Iterations need no barrier between them: a lane's last LDS reads (the
 // inverse's pass-0 gather) and its first LDS writes of the next transform
 // (the forward's pass-0 scatter) are the same positions of the same layout,
 // which no other lane touches in between.
 template<int N, int KIND>
-constexpr uint32_t conv_iters() { return (KIND == K_CONV && N == 16384) ? 8u : 1u; }
+constexpr bool conv_loops() { return KIND == K_CONV && N == 16384; }
+
+// The count is the launch's choice: a CU runs ceil(workgroups / CUs) of them
+// one after the other, iters transforms each, so the launch takes the iters
+// (at most 8) with the fewest transforms on the busiest CU, and among equals
+// the largest, which turns workgroups over least.  Up to 2048 transforms that
+// is one workgroup per CU.  Eight whatever the batch left a small one on a
+// few CUs: 99 transforms (13 workgroups) 118 us, 99 workgroups 17 us.
+inline uint32_t conv_iters(uint32_t ntrans)
+{
+   constexpr uint64_t CUS = 256, MOST = 8;
+   uint32_t best = 1;
+   uint64_t least = ~0ull;
+   for(uint64_t it = 1; it <= MOST; it++) {
+      const uint64_t wgs = (ntrans + it - 1) / it, load = (wgs + CUS - 1) / CUS * it;
+      if(load <= least) { least = load; best = (uint32_t)it; }
+   }
+   return best;
+}
 
 // A lane's V digit-order values (slots L*V + k of the transform at point
 // offset base) as 16-byte pairs: contiguous in digit order, at 2(L + m*T)
@@ -312,9 +330,13 @@ template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_kernel(const Conv1dParams p)
 {
-   constexpr uint32_t IT = conv_iters<N, KIND>();
+   if constexpr(conv_loops<N, KIND>()) {
 #pragma unroll 1
-   for(uint32_t it = 0; it < IT; it++) conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x * IT + it);
+      for(uint32_t it = 0; it < p.iters; it++)
+         conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x * p.iters + it);
+   } else {
+      conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x);
+   }
 }
 
 // the calls that read a filter, with a bperm filter
@@ -322,9 +344,13 @@ template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_bperm_kernel(const Conv1dParams p)
 {
-   constexpr uint32_t IT = conv_iters<N, KIND>();
+   if constexpr(conv_loops<N, KIND>()) {
 #pragma unroll 1
-   for(uint32_t it = 0; it < IT; it++) conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x * IT + it);
+      for(uint32_t it = 0; it < p.iters; it++)
+         conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x * p.iters + it);
+   } else {
+      conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x);
+   }
 }
 
 // (the XOR layout is a comparison option and has no bperm kernels)
@@ -353,9 +379,10 @@ static hipError_t launch_one(const Conv1dParams& p, hipStream_t s)
    if(!modulo_count_ok(p.fcount, p.ntrans) || !modulo_count_ok(p.scount, p.ntrans)) return hipErrorInvalidValue;
    static std::atomic<uint64_t> lds_ok[2]{};
    if(const hipError_t e = ensure_dynamic_lds(k, shm, lds_ok[bp]); e != hipSuccess) return e;
-   constexpr uint32_t IT = conv_iters<N, KIND>();
-   const dim3 grid((uint32_t)(((uint64_t)p.ntrans + CPB * IT - 1) / (CPB * IT))), block(CPB * T);
    Conv1dParams arg = p;
+   arg.iters = conv_loops<N, KIND>() ? conv_iters(p.ntrans) : 1;
+   const uint64_t per = (uint64_t)CPB * arg.iters;
+   const dim3 grid((uint32_t)((p.ntrans + per - 1) / per)), block(CPB * T);
    void* argv[] = { &arg };
    return hipLaunchKernel(k, grid, block, argv, shm, s);
 }

@@ -107,6 +107,7 @@ struct Conv1dParams {
    float         scale;    // K_PLAN_TAPS: factor applied to the spectrum
    uint32_t*     timing;   // K_CONV_TIMED: TIMER_STRIDE words per workgroup
    uint32_t      timing_groups;   // workgroups that write a record
+   uint32_t      iters;    // transforms per workgroup, in turn (set by the launcher; K_CONV at N = 16384)
 };
 
 bool       conv1d_supported(int n, int v);

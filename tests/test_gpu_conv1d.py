@@ -265,3 +265,27 @@ def test_config1_every_signal_against_fp64(dev):
                        * np.fft.fft(taps.astype(np.complex128))[None, :], axis=1)
     per = np.linalg.norm(got.reshape(batch, n) - want, axis=1) / np.linalg.norm(want, axis=1)
     assert O.rel_l2(got, want.reshape(-1)) <= TOL_F32 and per.max() <= 4 * TOL_F32
+
+
+@pytest.mark.parametrize("layout", ["dr", "bperm"])
+@pytest.mark.parametrize("batch", [1, 256, 257, 513, 2049])
+def test_16384_transforms_per_workgroup(dev, batch, layout):
+    """N = 16384: a workgroup runs 1 to 8 transforms in turn, the launch's choice
+    by the batch.  Every split gives what launches of one transform per
+    workgroup (at most 256 at a time) give, bit for bit, and writes nothing else."""
+    import torch
+    import fufft_amd as ff
+    n = 16384
+    print(f"case conv n={n} batch={batch} {layout}", flush=True)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(batch)
+    x = torch.randn(batch * n, dtype=torch.complex64, device=dev, generator=gen)
+    f = torch.randn(n, dtype=torch.complex64, device=dev, generator=gen)
+    out = torch.full(((batch + 1) * n,), 7.0 + 0j, dtype=torch.complex64, device=dev)
+    want = torch.empty_like(x)
+    ff.conv(x, f, out, n, batch, variant="v16", layout=layout)
+    for a in range(0, batch, 200):
+        b = min(batch, a + 200)
+        ff.conv(x[a * n: b * n], f, want[a * n: b * n], n, b - a, variant="v16", layout=layout)
+    assert torch.equal(torch.view_as_real(out[: batch * n]), torch.view_as_real(want))
+    assert bool((out[batch * n:] == 7.0).all())

@@ -1059,6 +1059,30 @@ int fufft_plan_filter_large_device_f32(const void* in, void* out, int64_t n, int
    return run_conv1d(K_PLAN_TAPS, mn, v, p, stream);
 }
 
+// How many of a batch's four-step transforms run the whole chain in one
+// workgroup each (radix-16 middle, n <= 32768), reading and writing the data
+// once where the three launches do it three times; the rest run those.  The
+// results are the same bit for bit, so the line is the faster side.  us a call,
+// shared filter, four buffers in turn, three launches / one:
+//   n =  8192: batch 1 12.7 / 9.8, 64 14.5 / 10.5, 256 23.6 / 12.7, 4096 241 / 124;
+//   n = 16384: 24 14.1 / 15.4, 48 17.0 / 16.4, 64 19.2 / 16.6, 128 25.4 / 17.6, 4096
+//     490 / 299;
+//   n = 32768: 80 34.4 / 35.5, 100 36.0 / 36.1, 128 39.4 / 38.4, 192 55.3 / 42.6,
+//     256 70.5 / 55.7, 512 131 / 107, 768 189 / 158, 4096 975 / 674.
+// At n = 32768 a transform fills a CU for some 32 us, so a last round of under
+// 100 of them is left to the three launches (530: 135 / 137, so 125), and one
+// full round with 32 or more behind it is not worth splitting (301: 81.3 / 87.9,
+// split 82.4).
+static int64_t chain_batch(int64_t n, int v, int64_t batch)
+{
+   if(!conv_chain_plan(n, v)) return 0;
+   if(n == 8192) return batch;
+   if(n == 16384) return batch >= 48 ? batch : 0;
+   const int64_t last = batch % 256;
+   if(last >= 100) return batch;
+   return batch < 512 && last >= 32 ? 0 : batch - last;
+}
+
 int fufft_conv_large_f32(void* buf, const void* filt, int64_t filt_stride, int64_t n,
                          int64_t batch, int mid, int variant, void* stream)
 {
@@ -1079,6 +1103,17 @@ int fufft_conv_large_f32(void* buf, const void* filt, int64_t filt_stride, int64
    if((st = current_table(&p.tw)) != FUFFT_OK) return st;
    if(batch == 0) return FUFFT_OK;
    hipStream_t s = static_cast<hipStream_t>(stream);
+   // the transforms that run the whole chain in one launch, then the others
+   const int64_t whole = lds_layout() == LAYOUT_XOR ? 0 : chain_batch(n, v, batch);
+   if(whole > 0) {
+      Conv1dParams q = p;
+      q.in0 = buf; q.out0 = buf; q.filt = filt;
+      q.ntrans = (uint32_t)whole; q.fcount = (uint32_t)(filt_stride == 0 ? 1 : whole);
+      q.scount = 1; q.mid = mid; q.fl = FUFFT_LAYOUT_DR;
+      st = n == CONV_WIDE_N ? status_of(launch_conv_wide_chain(q, (int)n, s))
+                            : run_conv1d(K_CONV_CHAIN, (int)n, v, q, stream);
+      if(st != FUFFT_OK) return st;
+   }
    // The three stages run over sub-batches small enough for the data to stay
    // in the last-level cache from one stage to the next.  One filter per
    // transform streams a sub-batch's worth of filter bytes through the
@@ -1088,7 +1123,7 @@ int fufft_conv_large_f32(void* buf, const void* filt, int64_t filt_stride, int64
    // (a shared filter: 117.1 / 123.5 / 128.6 / 133.3 / 136.8), same box.
    const int64_t sub = subbatch_items(n * 8 * (filt_stride == n && mid_needs_filter(mid) ? 2 : 1), batch,
                                       SUBBATCH_FOURSTEP_MB);
-   for(int64_t t0 = 0; t0 < batch; t0 += sub) {
+   for(int64_t t0 = whole; t0 < batch; t0 += sub) {
       const int64_t nb = batch - t0 < sub ? batch - t0 : sub;
       float2* a = static_cast<float2*>(buf) + t0 * n;
       // forward outer levels, largest stride first

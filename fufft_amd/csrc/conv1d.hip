@@ -37,7 +37,7 @@ constexpr int cpb_for(int T) { return T >= 128 ? 1 : 256 / T; }
 // (the forward's pass-0 scatter) are the same positions of the same layout,
 // which no other lane touches in between.
 template<int N, int KIND>
-constexpr bool conv_loops() { return KIND == K_CONV && N == 16384; }
+constexpr bool conv_loops() { return (KIND == K_CONV || KIND == K_CONV_CHAIN) && N == 16384; }
 
 // The count is the launch's choice: a CU runs ceil(workgroups / CUs) of them
 // one after the other, iters transforms each, so the launch takes the iters
@@ -78,7 +78,8 @@ __device__ __forceinline__ void store_spectrum(const Buf& ob, const float2 (&r)[
 template<int N, int V, int LAYOUT, int KIND, int MID, bool BPERM>
 __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_t bid)
 {
-   using PL = Plan<N, V>;
+   constexpr bool CHAIN = KIND == K_CONV_CHAIN;
+   using PL = Plan<N, V, V, CHAIN>;
    using LD = Lds<V, LAYOUT>;
    constexpr int T     = PL::T;
    constexpr int CPB   = cpb_for(T);
@@ -106,9 +107,8 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // the signal read and the result written once per launch stream past the
    // caches in the single-launch conv and C2C; the four-step middle, the split
    // and 2D row kernels keep the default policy
-   constexpr int  IO_POL    = (KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || TIMED || C2C_FWD ||
-                               C2C_INV) ? POL_NT
-                                                                                              : POL_DEFAULT;
+   constexpr int  IO_POL    = (KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED ||
+                               C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
    constexpr int  EL_IN     = REAL_IN ? 4 : 8;
    constexpr int  EL_OUT    = REAL_OUT ? 4 : 8;
 
@@ -417,6 +417,13 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
          // middle) or radix 8
          if constexpr(N >= 512 && N <= 4096) return launch_mid<N, V, LAYOUT, K_CONV_MID>(p, s);
          else                                return hipErrorInvalidValue;
+      case K_CONV_CHAIN:
+         // digit-order (chain-order) filters only, default LDS layouts
+         if constexpr(conv_chain_plan(N, V) && N < CONV_WIDE_N && LAYOUT != LAYOUT_XOR) {
+            return p.fl == FLT_DR ? launch_mid<N, V, LAYOUT, K_CONV_CHAIN>(p, s) : hipErrorInvalidValue;
+         } else {
+            return hipErrorInvalidValue;
+         }
       case K_CONV_R2: return launch_one<N, V, LAYOUT, K_CONV_R2, MID_MUL>(p, s);
       case K_FWD:     return launch_one<N, V, LAYOUT, K_FWD, MID_NONE>(p, s);
       case K_APPLY:   return launch_mid<N, V, LAYOUT, K_APPLY>(p, s);

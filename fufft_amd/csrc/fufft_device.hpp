@@ -195,30 +195,38 @@ __device__ __forceinline__ float2 tw_load(const float2* __restrict__ tw, int idx
 // The forms below (the single chain's state in pw, the parity chains'
 // running pair) are the ones the kernels were measured with: other forms of
 // the same recurrences schedule differently, up to 1.5% slower.
-template<int R, int OFF, int STRIDE, int NR>
+// COUNT neighbouring groups (offsets OFF, OFF + 1, ...) that share W^j take
+// each power as it is made, so the chain runs once for all of them.
+template<int R, int OFF, int STRIDE, int COUNT = 1, int NR>
 __device__ __forceinline__ void chain_one(float2 (&r)[NR], float2 w1, float2 (&pw)[R])
 {
    pw[1] = w1;
-   r[OFF + STRIDE] = cmul(r[OFF + STRIDE], w1);
+#pragma unroll
+   for(int g = 0; g < COUNT; g++) r[OFF + g + STRIDE] = cmul(r[OFF + g + STRIDE], w1);
 #pragma unroll
    for(int k = 2; k < R; k++) {
       pw[k] = cmul(pw[k - 1], w1);
-      r[OFF + k * STRIDE] = cmul(r[OFF + k * STRIDE], pw[k]);
+#pragma unroll
+      for(int g = 0; g < COUNT; g++) r[OFF + g + k * STRIDE] = cmul(r[OFF + g + k * STRIDE], pw[k]);
    }
 }
 
-template<int OFF, int STRIDE, bool KEEP, int NR>
+template<int OFF, int STRIDE, bool KEEP, int COUNT = 1, int NR>
 __device__ __forceinline__ void chain_parity(float2 (&r)[NR], float2 w1, float2 (&pw)[16])
 {
    const float2 sq = cmul(w1, w1);
    if constexpr(KEEP) { pw[1] = w1; pw[2] = sq; }
-   r[OFF + STRIDE] = cmul(r[OFF + STRIDE], w1);
+#pragma unroll
+   for(int g = 0; g < COUNT; g++) r[OFF + g + STRIDE] = cmul(r[OFF + g + STRIDE], w1);
    float2 run[2] = {sq, cmul(sq, w1)};   // the powers of the even and odd taps
    if constexpr(KEEP) pw[3] = run[1];
 #pragma unroll
    for(int m = 1; m < 8; m++) {
 #pragma unroll
-      for(int q = 0; q < 2; q++) r[OFF + (2 * m + q) * STRIDE] = cmul(r[OFF + (2 * m + q) * STRIDE], run[q]);
+      for(int q = 0; q < 2; q++)
+#pragma unroll
+         for(int g = 0; g < COUNT; g++)
+            r[OFF + g + (2 * m + q) * STRIDE] = cmul(r[OFF + g + (2 * m + q) * STRIDE], run[q]);
       if(m < 7) {
 #pragma unroll
          for(int q = 0; q < 2; q++) run[q] = cmul(run[q], sq);
@@ -246,12 +254,12 @@ __device__ __forceinline__ void tw_kept_conj(float2 (&r)[NR], const float2 (&w)[
 // chain, as the reference's kernels do
 enum { CHAIN_SINGLE = 0, CHAIN_EVENODD = 1 };
 
-template<int R, int CHAIN, int OFF, int STRIDE, int NR>
+template<int R, int CHAIN, int OFF, int STRIDE, int COUNT = 1, int NR>
 __device__ __forceinline__ void twiddle_group(float2 (&r)[NR], float2 w1)
 {
    float2 pw[R];
-   if constexpr(R == 16 && CHAIN == CHAIN_EVENODD) chain_parity<OFF, STRIDE, false>(r, w1, pw);
-   else                                             chain_one<R, OFF, STRIDE>(r, w1, pw);
+   if constexpr(R == 16 && CHAIN == CHAIN_EVENODD) chain_parity<OFF, STRIDE, false, COUNT>(r, w1, pw);
+   else                                             chain_one<R, OFF, STRIDE, COUNT>(r, w1, pw);
 }
 
 // ---- buffer-resource memory access ---------------------------------------------------

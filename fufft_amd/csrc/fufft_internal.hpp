@@ -57,13 +57,16 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 // K_CONV_PSF: K_CONV for one lane-major filter per signal at radix 16,
 // N = 4096: the filter loads go out with the signal loads (without the kept
 // twiddle chain, for the registers they hold through the forward DIF).
+// K_CONV_CHAIN: the four-step chain of one outer level (a radix-16 pass with the
+// single twiddle chain, then the middle's plan) in one workgroup, for a filter
+// in the chain order.
 // K_CONV_PSF_DR: the same for one digit-order filter per signal (the
 // reference's own per-signal format): the loads of each wavefront's 1 KiB
 // filter runs go out with the signal loads, the hand-off to the lanes goes
 // through LDS at the mid operation.
 enum { K_CONV = 0, K_CONV_R2 = 1, K_FWD = 2, K_APPLY = 3, K_FWD_R2 = 4, K_APPLY_R2 = 5,
        K_C2C_FWD = 6, K_C2C_INV = 7, K_PLAN_TAPS = 8, K_CONV_TIMED = 9, K_CONV_MID = 10,
-       K_CONV_PSF = 11, K_CONV_PSF_DR = 12 };
+       K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13 };
 
 // the plans K_CONV_PSF and K_CONV_PSF_DR are built for: radix 16 with whole
 // wavefronts per transform and room for the filter's 32 VGPRs within 128
@@ -128,6 +131,13 @@ constexpr bool conv_wide_plan(int64_t n, int v) { return n == CONV_WIDE_N && v =
 // 196.8, so those keep the workgroup kernel.
 constexpr bool conv_wide_shared_lane_plan(int64_t n, int v) { return n == 16384 && v == 16; }
 hipError_t launch_conv_wide(const Conv1dParams& p, int n, hipStream_t s);
+
+// The four-step chain of one outer level in one launch: K_CONV_CHAIN at
+// N = 8192 and 16384, the wide kernel at 32768.  Against the three launches:
+// 8192 x 4000 248.9 -> 124.8 us, 16384 x 300 43.4 -> 36.2, 32768 x 256 68.5 ->
+// 52.5; the batches that take it are chain_batch's choice (capi.hip).
+constexpr bool conv_chain_plan(int64_t n, int v) { return v == 16 && (n == 8192 || n == 16384 || n == CONV_WIDE_N); }
+hipError_t launch_conv_wide_chain(const Conv1dParams& p, int n, hipStream_t s);
 
 // ---- filter planning on the device (plan.hip) ----------------------------------------
 struct GatherDigits {

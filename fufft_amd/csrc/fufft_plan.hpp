@@ -31,19 +31,27 @@ constexpr int ilog2c(int x) { int r = 0; while((1 << r) < x) r++; return r; }
 
 // RM is the radix of the main passes, V by default; with V = 2 * RM every lane
 // runs two groups of each main pass (the 32-values-per-lane conv, wide.hip).
-template<int N_, int V_, int RM_ = V_>
+// CHAIN: the four-step chain of one outer level in one workgroup, a radix-16
+// pass (the outer level's single twiddle chain) before the passes of N/16.
+template<int N_, int V_, int RM_ = V_, bool CHAIN_ = false>
 struct Plan {
    static constexpr int N = N_, V = V_, RM = RM_;
+   static constexpr bool CHAIN = CHAIN_;
    static constexpr int LOGN = ilog2c(N), LOGV = ilog2c(V), LOGR = ilog2c(RM);
-   static constexpr int NR   = LOGN / LOGR;
-   static constexpr int LEAD = 1 << (LOGN % LOGR);
-   static constexpr int NP   = NR + (LEAD > 1 ? 1 : 0);
+   static constexpr int LOGI = LOGN - (CHAIN ? 4 : 0);      // the plan after the outer level
+   static constexpr int NR   = LOGI / LOGR;
+   static constexpr int LEAD = 1 << (LOGI % LOGR);
+   static constexpr int NP   = NR + (LEAD > 1 ? 1 : 0) + (CHAIN ? 1 : 0);
    static constexpr int T    = N / V;
    static_assert((1 << LOGN) == N && (1 << LOGV) == V && (1 << LOGR) == RM, "power-of-two sizes only");
    static_assert(NR >= 1, "N must hold at least one main pass");
    static_assert(V % RM == 0 && V % LEAD == 0, "whole groups per lane");
 
-   static constexpr int radix(int p) { return (LEAD > 1 && p == 0) ? LEAD : RM; }
+   static constexpr int radix(int p)
+   {
+      if(CHAIN && p == 0) return 16;
+      return (LEAD > 1 && p == (CHAIN ? 1 : 0)) ? LEAD : RM;
+   }
    static constexpr int stride(int p)
    {
       int M = N;
@@ -212,15 +220,21 @@ __device__ __forceinline__ void lds_scatter(const float2 (&r)[PL::V], float2* A,
 // cache line, and the vector-memory path, not the VALU, becomes the limit.)
 // Base twiddles depend only on the lane, so all of them are read once at
 // kernel start: (cos, sin)(2*pi*j/P) serves the forward pass as (c, -s) and
-// the inverse pass as (c, s).  Slot numbering: passes with M > 1 in order,
-// G_p slots each.
+// the inverse pass as (c, s).  Group g of pass p has j = (L + g*T) mod M, which
+// repeats after M/T groups: at M <= T every group shares one W^j.  Slot
+// numbering: passes with M > 1 in order, one slot per distinct j.
 template<class PL>
 struct Twiddles {
+   static constexpr int distinct(int p)
+   {
+      const int g = PL::V / PL::radix(p), m = PL::stride(p) / PL::T;
+      return m < 1 ? 1 : m < g ? m : g;
+   }
    static constexpr int slots_before(int p)
    {
       int n = 0;
       for(int i = 0; i < p; i++)
-         if(PL::stride(i) > 1) n += PL::V / PL::radix(i);
+         if(PL::stride(i) > 1) n += distinct(i);
       return n;
    }
    static constexpr int COUNT = slots_before(PL::NP) > 0 ? slots_before(PL::NP) : 1;
@@ -230,10 +244,10 @@ struct Twiddles {
    template<int p>
    __device__ __forceinline__ void load_pass(const Buf& tb, int L)
    {
-      constexpr int R = PL::radix(p), M = PL::stride(p), G = PL::V / R;
+      constexpr int R = PL::radix(p), M = PL::stride(p);
       if constexpr(M > 1) {
 #pragma unroll
-         for(int g = 0; g < G; g++)
+         for(int g = 0; g < distinct(p); g++)
             w[slots_before(p) + g] = tb.ld2((uint32_t)(((L + g * PL::T) & (M - 1)) * 8), R * M * 8);
       }
    }
@@ -280,16 +294,24 @@ enum { KEEP_NONE = 0, KEEP_STORE = 1, KEEP_USE = 2 };
 template<class PL, int P, int SIGN, bool DIT, int KEEP = KEEP_NONE>
 __device__ __forceinline__ void compute_pass(float2 (&r)[PL::V], const Twiddles<PL>& tw, KeptChain<PL>& kc)
 {
-   constexpr int R = PL::radix(P), M = PL::stride(P), G = PL::V / R;
+   constexpr int R = PL::radix(P), M = PL::stride(P), G = PL::V / R, D = Twiddles<PL>::distinct(P);
    constexpr bool keep = KeptChain<PL>::enabled && P == KeptChain<PL>::P && KEEP != KEEP_NONE;
-   static_for<G>([&](auto gi) {
+   constexpr int CH = PL::CHAIN && P == 0 ? CHAIN_SINGLE : CHAIN_EVENODD;
+   if constexpr(M > 1 && G > 1 && D == 1) {
+      // one W^j for all groups: the chain runs once
+      const float2 b = tw.w[Twiddles<PL>::slots_before(P)];
+      const float2 w1 = SIGN < 0 ? make_float2(b.x, -b.y) : b;
+      if constexpr(DIT) twiddle_group<R, CH, 0, G, G>(r, w1);
+      static_for<G>([&](auto gi) { dftR<R, SIGN, decltype(gi)::value, G>(r); });
+      if constexpr(!DIT) twiddle_group<R, CH, 0, G, G>(r, w1);
+   } else static_for<G>([&](auto gi) {
       constexpr int g = decltype(gi)::value;
       if constexpr(M > 1) {
-         const float2 b = tw.w[Twiddles<PL>::slots_before(P) + g];
+         const float2 b = tw.w[Twiddles<PL>::slots_before(P) + g % D];
          const float2 w1 = SIGN < 0 ? make_float2(b.x, -b.y) : b;
          if constexpr(DIT) {
             if constexpr(keep && KEEP == KEEP_USE) tw_kept_conj<R, g, G>(r, kc.w);
-            else                                   twiddle_group<R, CHAIN_EVENODD, g, G>(r, w1);
+            else                                   twiddle_group<R, CH, g, G>(r, w1);
          }
          dftR<R, SIGN, g, G>(r);
          if constexpr(!DIT) {
@@ -297,7 +319,7 @@ __device__ __forceinline__ void compute_pass(float2 (&r)[PL::V], const Twiddles<
                if constexpr(R == 16) chain_parity<g, G, true>(r, w1, kc.w);
                else                  chain_one<R, g, G>(r, w1, kc.w);
             }
-            else                                     twiddle_group<R, CHAIN_EVENODD, g, G>(r, w1);
+            else                                     twiddle_group<R, CH, g, G>(r, w1);
          }
       } else {
          dftR<R, SIGN, g, G>(r);

@@ -39,6 +39,18 @@
 // digit-order one, against 135-138 for the four-step chain at the same N (48
 // bytes per point over HBM and the Infinity Cache).
 //
+// A lane's groups of the later passes share one W^j (M <= 1024 lanes), so each
+// of those passes runs its twiddle chain once for both groups: 649.6 -> 633.3 us
+// (lane-major), 693.0 -> 682.7 (digit order), N = 16384 573.5 -> 552.1, 2^27 or
+// 2^26 points, bit-identical.
+//
+// The four-step chain at N = 32768 (CHAIN: radix 16 with the single twiddle
+// chain, then LEAD 8 and two radix-16 passes) is the same kernel with its passes
+// in that order, for a filter in the chain order: one read and one write of the
+// data where fufft_conv_large_f32's three launches make three of each.  1000
+// transforms 244 -> 191 us; which batches take it is chain_batch's choice
+// (capi.hip).
+//
 // N = 16384 runs the same code with 512 lanes (LEAD 4, eight groups per lane
 // in the lead pass): 68 KiB of LDS, so two workgroups share a CU and one's
 // loads overlap the other's passes.  fufft_conv_f32 takes it for a shared
@@ -51,8 +63,8 @@ namespace fufft {
 
 namespace {
 
-template<int N>
-using WPlan = Plan<N, 32, 16>;
+template<int N, bool CHAIN = false>
+using WPlan = Plan<N, 32, 16, CHAIN>;
 
 // Float slot layouts.  gfx950 serves the 4-byte LDS forms 32 lanes at a time
 // over 32 banks (bank = slot mod 32), each access of a paired form
@@ -200,11 +212,11 @@ __device__ __forceinline__ void wide_mid(float2 (&r)[PL::V], const Buf& fb, uint
    }
 }
 
-template<int N_, int MID, int FLT>
+template<int N_, int MID, int FLT, bool CHAIN>
 __global__ void __launch_bounds__(WPlan<N_>::T, 4)
 conv_wide_kernel(const Conv1dParams p)
 {
-   using PL = WPlan<N_>;
+   using PL = WPlan<N_, CHAIN>;
    constexpr int N = PL::N, T = PL::T, V = PL::V;
    extern __shared__ float ldsf[];
    const int L = threadIdx.x;
@@ -235,13 +247,13 @@ conv_wide_kernel(const Conv1dParams p)
    // read again for the inverse's lead pass (from the cache), they are free
    // in between, and the kernel fits 128 VGPRs with no scratch (48-68 bytes
    // per lane when held throughout).
-   constexpr bool RELOAD_LEAD = PL::V / PL::radix(0) > 4;
+   constexpr bool RELOAD_LEAD = Twiddles<PL>::distinct(0) > 4;
    static_for<PL::NP>([&](auto qi) {
       constexpr int P = PL::NP - 1 - decltype(qi)::value;
       if constexpr(RELOAD_LEAD && P == 0) {
          tw.template load_pass<0>(Buf(p.tw, FUFFT_TW_ENTRIES * 8u), L);
 #pragma unroll
-         for(int i = 0; i < PL::V / PL::radix(0); i++) asm volatile("" : "+v"(tw.w[i].x), "+v"(tw.w[i].y));
+         for(int i = 0; i < Twiddles<PL>::distinct(0); i++) asm volatile("" : "+v"(tw.w[i].x), "+v"(tw.w[i].y));
       }
       compute_pass<PL, P, +1, true, KEEP_NONE>(r, tw, kc);
       if constexpr(P > 0) split_exchange<PL, P, P - 1>(r, ldsf, L);
@@ -251,10 +263,10 @@ conv_wide_kernel(const Conv1dParams p)
    for(int q = 0; q < V; q++) ob.st2<POL_NT>(r[q], (uint32_t)L * 8u, q * T * 8);
 }
 
-template<int N, int MID, int FLT>
+template<int N, int MID, int FLT, bool CHAIN>
 hipError_t launch_wide_mid(const Conv1dParams& p, hipStream_t s)
 {
-   const void* k = reinterpret_cast<const void*>(&conv_wide_kernel<N, MID, FLT>);
+   const void* k = reinterpret_cast<const void*>(&conv_wide_kernel<N, MID, FLT, CHAIN>);
    constexpr size_t shm = (size_t)Pad16::size(N) * sizeof(float);
    static std::atomic<uint64_t> lds_ok{};
    if(const hipError_t e = ensure_dynamic_lds(k, shm, lds_ok); e != hipSuccess) return e;
@@ -268,7 +280,7 @@ hipError_t launch_wide_mid(const Conv1dParams& p, hipStream_t s)
 // Per-signal filters address with 32-bit byte offsets: beyond 4 GiB of them
 // the launch is split into chunks of transforms (signal, result and filter
 // advance together).
-template<int N>
+template<int N, bool CHAIN>
 hipError_t launch_conv_wide_n(const Conv1dParams& p, hipStream_t s)
 {
    if(p.ntrans == 0) return hipSuccess;
@@ -277,9 +289,14 @@ hipError_t launch_conv_wide_n(const Conv1dParams& p, hipStream_t s)
    auto one = [&](const Conv1dParams& q) {
       return with_mid(q.mid, [&](auto m) {
          constexpr int MID = decltype(m)::value;
-         if constexpr(!mid_reads_filter<MID>) return launch_wide_mid<N, MID, FLT_DR>(q, s);
-         else return q.fl == FLT_LANE ? launch_wide_mid<N, MID, FLT_LANE>(q, s)
-                   : q.fl == FLT_BPERM ? launch_wide_mid<N, MID, FLT_BPERM>(q, s) : launch_wide_mid<N, MID, FLT_DR>(q, s);
+         if constexpr(CHAIN || !mid_reads_filter<MID>) {
+            return !mid_reads_filter<MID> || q.fl == FLT_DR ? launch_wide_mid<N, MID, FLT_DR, CHAIN>(q, s)
+                                                            : hipErrorInvalidValue;
+         } else {
+            return q.fl == FLT_LANE  ? launch_wide_mid<N, MID, FLT_LANE, false>(q, s)
+                 : q.fl == FLT_BPERM ? launch_wide_mid<N, MID, FLT_BPERM, false>(q, s)
+                                     : launch_wide_mid<N, MID, FLT_DR, false>(q, s);
+         }
       });
    };
    constexpr uint64_t bytes = (uint64_t)N * 8;
@@ -300,9 +317,14 @@ hipError_t launch_conv_wide_n(const Conv1dParams& p, hipStream_t s)
 
 hipError_t launch_conv_wide(const Conv1dParams& p, int n, hipStream_t s)
 {
-   if(n == CONV_WIDE_N) return launch_conv_wide_n<CONV_WIDE_N>(p, s);
-   if(n == 16384)       return launch_conv_wide_n<16384>(p, s);
+   if(n == CONV_WIDE_N) return launch_conv_wide_n<CONV_WIDE_N, false>(p, s);
+   if(n == 16384)       return launch_conv_wide_n<16384, false>(p, s);
    return hipErrorInvalidValue;
+}
+
+hipError_t launch_conv_wide_chain(const Conv1dParams& p, int n, hipStream_t s)
+{
+   return n == CONV_WIDE_N ? launch_conv_wide_n<CONV_WIDE_N, true>(p, s) : hipErrorInvalidValue;
 }
 
 }  // namespace fufft

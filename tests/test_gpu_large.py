@@ -106,3 +106,38 @@ def test_large_rejects_bad_args(dev):
         ff.check(ff.lib.fufft_conv_large_f32(buf.data_ptr(), buf.data_ptr(), 0, 8192, 1, 0, 9, None),
                  "fufft_conv_large_f32")
     ff.conv_large(buf, buf, n=8192, batch=0)                # empty batch is a no-op
+
+
+@pytest.mark.parametrize("own_filters", [False, True])
+@pytest.mark.parametrize("n,batch", [(8192, 1), (8192, 257), (16384, 47), (16384, 48), (16384, 513), (32768, 99),
+                                     (32768, 100), (32768, 257), (32768, 287), (32768, 288), (32768, 356),
+                                     (32768, 513)])
+def test_large_split_between_one_launch_and_three(dev, n, batch, own_filters):
+    """Up to n = 32768 the batch decides how many transforms run the chain in one
+    workgroup and how many in three launches.  On both sides of every line the
+    result is what the same transforms give in other batches, bit for bit
+    (their own parity: test_large_matches_oracle and the sampled ones below),
+    and nothing behind the batch is written."""
+    import torch
+    import fufft_amd as ff
+    print(f"case large split n={n} batch={batch} own_filters={own_filters}", flush=True)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(n + batch)
+    x = torch.randn(batch * n, dtype=torch.complex64, device=dev, generator=gen)
+    spec = torch.randn(n * (batch if own_filters else 1), dtype=torch.complex64, device=dev, generator=gen)
+    f = torch.empty_like(spec)
+    ff.plan_filter_large_device(spec, f, n, count=f.numel() // n)
+    buf = torch.cat([x, torch.full((n,), 7.0 + 0j, dtype=torch.complex64, device=dev)])
+    ff.conv_large(buf, f, n, batch, filt_stride=n if own_filters else 0)
+    want = x.clone()
+    for a in range(0, batch, 40):                     # three launches at 16384 and 32768, one at 8192
+        b = min(batch, a + 40)
+        ff.conv_large(want[a * n: b * n], f[a * n: b * n] if own_filters else f, n, b - a,
+                      filt_stride=n if own_filters else 0)
+    assert torch.equal(torch.view_as_real(buf[: batch * n]), torch.view_as_real(want))
+    assert bool((buf[batch * n:] == 7.0).all())
+    # the first and last transforms against the oracle
+    for t in (0, batch - 1):
+        ft = f.view(-1, n)[t if own_filters else 0].cpu().numpy()
+        assert bits_equal(buf[t * n: (t + 1) * n].cpu().numpy(),
+                          O.conv(x[t * n: (t + 1) * n].cpu().numpy(), ft, n, oracle_plan(n)))

@@ -25,9 +25,48 @@
 
 namespace fufft {
 
-// values per lane and columns per workgroup for a column length h
+// values per lane for a column length h, and the most columns a workgroup of
+// 1024 lanes takes
 constexpr int col_v(int h) { return h <= 512 ? 8 : 16; }
-constexpr int col_c(int h) { return (1024 / (h / col_v(h))) < 16 ? 1024 / (h / col_v(h)) : 16; }
+constexpr int col_most(int h) { return h <= 1024 ? 16 : 8; }
+
+// Points of a split apply from which its filters are streamed (below they come
+// back from the last-level cache in the next call: 2048 x 2048 56.8 us, 62.7
+// streamed; 8 M points 103 and 98).
+constexpr uint64_t kApplyStream = 1u << 22;
+
+// Columns per workgroup, 16, 8 or 4, by the launch's points.  16 columns make
+// every tap a whole 128-byte line, 8 and 4 make more and smaller workgroups of
+// the same work.  us a call, 4 / 8 / 16 columns:
+//   conv, h = 256: 65 K points 12.0 / 13.2 / 13.3, 1 M 18.3 / 17.6 / 18.0, 4 M 41 / 38 /
+//     37, 33 M 315 / 283 / 269;
+//   h = 512: 262 K 12.7 / 13.5 / 15.1, 1 M 17.2 / 17.1 / 18.2, 2.4 M 29.0 / 27.7 / 28.9,
+//     8 M 82.6 / 74.4 / 75.6, 33 M 310 / 288 / 279;
+//   h = 1024 (16 columns fill a CU's LDS): 524 K 17.5 / 18.6 / 22.1, 2.4 M 27.0 / 26.7 /
+//     28.5, 33 M 334 / 296 / 311;
+//   h = 2048: 524 K 20.5 / 23.9, 4 M 50.7 / 46.1, 33 M 435 / 361.
+// The split apply reads a filter per image once, which favours whole lines
+// sooner: h = 512, 2.4 M 26.8 / 25.6 / 30.2, 8 M 64 / 62 / 61, 33 M 236 / 237 / 204;
+// h = 1024, 2.4 M 28.6 / 27.9 / 34.5, 8 M 83 / 74 / 66.
+static int col_width(int kind, int h, uint64_t points)
+{
+   const bool lines = kind == COL_APPLY ? h <= 1024 && points > kApplyStream
+                                                : h <= 512 && points > (uint64_t)h * 16384;
+   if(lines) return 16;
+   return points >= (uint64_t)h * 8 * 200 ? 8 : 4;
+}
+
+// Column tile of a workgroup.  Workgroups go to the 8 XCDs in turn, so the
+// SHARE = 16 / C tiles that share their 128-byte lines are given to SHARE
+// workgroups of one XCD, 8 apart, and meet in its L2: h = 2048 (C = 8), 33 M
+// points 434 -> 361 us.  A launch has a multiple of 8 * SHARE tiles (rows are at
+// least 256 points).
+template<uint32_t SHARE>
+__device__ __forceinline__ uint32_t col_tile(uint32_t b)
+{
+   const uint32_t in = b % (8 * SHARE);
+   return b - in + (in % 8) * SHARE + in / 8;
+}
 
 template<int H, int V, int LAYOUT, int KIND, int MID, int C>
 __global__ void __launch_bounds__(C * (H / V)) col_kernel(const ColParams p)
@@ -41,8 +80,9 @@ __global__ void __launch_bounds__(C * (H / V)) col_kernel(const ColParams p)
    const int col = threadIdx.x % C;
    const int L   = threadIdx.x / C;
    const uint32_t tiles = p.w / C;
-   const uint32_t img   = blockIdx.x / tiles;
-   const uint32_t c     = (blockIdx.x - img * tiles) * C + col;
+   const uint32_t tile  = col_tile<16 / C>(blockIdx.x);
+   const uint32_t img   = tile / tiles;
+   const uint32_t c     = (tile - img * tiles) * C + col;
    const uint32_t W8    = p.w * 8u;
    const uint32_t ibytes = (uint32_t)H * W8;
    const uint32_t nat = (uint32_t)L * W8 + c * 8u;           // row L, column c
@@ -83,8 +123,8 @@ __global__ void __launch_bounds__(C * (H / V)) col_kernel(const ColParams p)
          // columns are scattered over the row, its cache lines are shared
          // with other tiles, and NT cost 4.5%.
          if constexpr(KIND == COL_APPLY) {
-            if(!p.f_dr && p.fcount == p.nimg) mid_op<PL, MID, POL_NT>(r, fb, fo, W8);
-            else                              mid_op<PL, MID>(r, fb, fo, W8);
+            if(p.f_stream) mid_op<PL, MID, POL_NT>(r, fb, fo, W8);
+            else           mid_op<PL, MID>(r, fb, fo, W8);
          } else {
             mid_op<PL, MID>(r, fb, fo, W8);
          }
@@ -95,23 +135,34 @@ __global__ void __launch_bounds__(C * (H / V)) col_kernel(const ColParams p)
    }
 }
 
-template<int H, int KIND, int MID>
-static hipError_t launch_col_one(const ColParams& p, hipStream_t s)
+template<int H, int KIND, int MID, int C>
+static hipError_t launch_col_tiles(const ColParams& p, hipStream_t s)
 {
-   constexpr int V = col_v(H), T = H / V, C = col_c(H);
+   constexpr int V = col_v(H), T = H / V;
    constexpr int SLOTC = Lds<V, LAYOUT_PAD>::size(H) + 16 / C;
    const size_t shm = (size_t)C * SLOTC * sizeof(float2);
    const void* k = reinterpret_cast<const void*>(&col_kernel<H, V, LAYOUT_PAD, KIND, MID, C>);
    static std::atomic<uint64_t> lds_ok{0};
    if(const hipError_t e = ensure_dynamic_lds(k, shm, lds_ok); e != hipSuccess) return e;
-   if(p.w % C || !modulo_count_ok(p.fcount, p.nimg) || !modulo_count_ok(p.scount, p.nimg))
+   if(p.w % 128 || !modulo_count_ok(p.fcount, p.nimg) || !modulo_count_ok(p.scount, p.nimg))
       return hipErrorInvalidValue;
    const uint64_t blocks = (uint64_t)p.nimg * (p.w / C);
    if(blocks > 0x7fffffffu) return hipErrorInvalidValue;
    const dim3 grid((unsigned)blocks), block(C * T);
    ColParams arg = p;
+   arg.f_stream = KIND == COL_APPLY && !p.f_dr && p.fcount == p.nimg && (uint64_t)p.nimg * H * p.w > kApplyStream;
    void* argv[] = { &arg };
    return hipLaunchKernel(k, grid, block, argv, shm, s);
+}
+
+template<int H, int KIND, int MID>
+static hipError_t launch_col_one(const ColParams& p, hipStream_t s)
+{
+   switch(col_width(KIND, H, (uint64_t)p.nimg * H * p.w)) {
+      case 4:  return launch_col_tiles<H, KIND, MID, 4>(p, s);
+      case 8:  return launch_col_tiles<H, KIND, MID, 8>(p, s);
+      default: return launch_col_tiles<H, KIND, MID, col_most(H)>(p, s);
+   }
 }
 
 template<int H, int KIND>

@@ -234,6 +234,7 @@ struct ColParams {
    uint32_t      f_dr;
    uint32_t      f_tr_log;
    uint32_t      f_vr_log;
+   uint32_t      f_stream; // COL_APPLY: read the filters past the caches (set by the launcher)
 };
 enum { COL_CONV = 0, COL_FWD = 1, COL_APPLY = 2 };
 int        col_values_per_lane(int h);      // 0 if h is not a supported column length

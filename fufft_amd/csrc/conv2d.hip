@@ -201,17 +201,40 @@ int col_values_per_lane(int h)
 // at lane i % TW (TW = W/8), in the column phases column i / TH at lane i % TH
 // (TH = H/8); both are at most 64, so each row or column transform lies inside
 // one wavefront and its exchanges need a wavefront fence only.  Between the
-// phases the image crosses LDS transposed (columns contiguous, one spare slot
-// per column); workgroup barriers order those crossings.  Images past the
-// batch run on empty buffer ranges (loads return zero, stores are dropped), so
-// every lane meets every barrier.
+// phases the image crosses LDS transposed (Turn below); workgroup barriers order
+// those crossings.  Images past the batch run on empty buffer ranges (loads
+// return zero, stores are dropped), so every lane meets every barrier.
 constexpr int small2d_lanes(int h, int w) { return h * w / 8; }
 constexpr int small2d_images(int h, int w) { return small2d_lanes(h, w) >= 256 ? 1 : 256 / small2d_lanes(h, w); }
 constexpr int small2d_slot(int h, int w)
 {
-   const int rows = h * (w + w / 8), cols = w * (h + h / 8), tr = w * (h + 1);
-   return rows > cols ? (rows > tr ? rows : tr) : (cols > tr ? cols : tr);
+   return h * w + h * w / 8;                       // h rows of w + w/8 slots, or w columns of h + h/8
 }
+
+// LDS slot of the image between the phases: entry (s, r), row r's spectrum slot
+// s, in column s's own SH = H + H/8 slots, at r with some of its low four bits
+// flipped.  16 lanes of a row phase hold neighbouring slots 8 apart (bits 3.. of
+// s) of neighbouring rows (bits 0.. of r): the flip moves the former onto the
+// bits of r that the latter leave, and both sides of both crossings touch 16
+// residues modulo 16 (a column phase's neighbouring s fall apart by SH).  With a
+// spare slot per column instead, the row side met 4 to 8 lanes to a bank.  A
+// column's slots are its own wavefront's in every column phase, so its lanes
+// pass from the crossing to their exchanges, and back, without a barrier (4 per
+// image instead of 6).  33 M points, us: 64 x 64 125 -> 109, 64 x 128 249 -> 156, 32 x
+// 256 195 -> 152, 16 x 512 168 -> 138, 8 x 256 129 -> 104, 128 x 64 162 -> 150, 512 x 16
+// 222 -> 173; rows of 8 and 16 points, which had no such conflicts, within 1.3%.
+template<int H, int W>
+struct Turn {
+   static constexpr int SH = H + H / 8;
+   static constexpr int lanes = ilog2c(W / 8) < 4 ? ilog2c(W / 8) : 4;
+   // at H = 8 the lowest of those bits already moves SH * 8 = 72 slots: 8 modulo 16
+   static constexpr int from = H == 8 ? 4 : 3, bits = H == 8 ? (lanes > 0 ? lanes - 1 : 0) : lanes;
+   static constexpr int to = (H == 8 ? 3 : 4) - bits;
+   static __host__ __device__ constexpr int slot(int s, int r)
+   {
+      return s * SH + (r ^ (((s >> from) & ((1 << bits) - 1)) << to));
+   }
+};
 
 template<int H, int W, int MID>
 __global__ void __launch_bounds__(small2d_images(H, W) * small2d_lanes(H, W))
@@ -222,9 +245,13 @@ small2d_kernel(const Small2dParams p)
    using LD = Lds<8, LAYOUT_PAD>;
    using Op = MidOf<MID>;
    constexpr int TW = W / 8, TH = H / 8, I = small2d_lanes(H, W), IPB = small2d_images(H, W);
-   constexpr int SW = LD::size(W), SH = LD::size(H), CT = H + 1, SLOT = small2d_slot(H, W);
+   using TN = Turn<H, W>;
+   constexpr int SW = LD::size(W), SH = LD::size(H), SLOT = small2d_slot(H, W);
+   static_assert(SH == TN::SH, "one region per column");
    constexpr uint32_t BYTES = H * W * 8;
    static_assert(TW <= 64 && TH <= 64, "a row or column transform inside one wavefront");
+   constexpr int KEEP_F = H * W <= 4096 ? KEEP_STORE : KEEP_NONE;
+   constexpr int KEEP_I = H * W <= 4096 ? KEEP_USE : KEEP_NONE;
 
    extern __shared__ float2 lds[];
    const int img = threadIdx.x / I, i = threadIdx.x % I;
@@ -284,17 +311,16 @@ small2d_kernel(const Small2dParams p)
       for(int q = 0; q < 8; q++) r[q] = ib.ld2((uint32_t)(rr * W + rl) * 8u, q * TW * 8);
    }
    forward_dif<PW, LD, 64>(r, S + rr * SW, rl, tww);
-   // transposed: row-spectrum slot s of row rr to S[s*CT + rr]
    __syncthreads();
 #pragma unroll
-   for(int k = 0; k < 8; k++) S[(rl * 8 + k) * CT + rr] = r[k];
+   for(int k = 0; k < 8; k++) S[TN::slot(rl * 8 + k, rr)] = r[k];
    __syncthreads();
    // columns DIF: lane (cc, cl) takes column cc's rows cl + q*TH
 #pragma unroll
-   for(int q = 0; q < 8; q++) r[q] = S[cc * CT + cl + q * TH];
-   __syncthreads();
+   for(int q = 0; q < 8; q++) r[q] = S[TN::slot(cc, cl + q * TH)];
+   pass_barrier<64>();
    KeptChain<PH> kc;
-   forward_dif<PH, LD, 64, 64, KEEP_STORE>(r, S + cc * SH, cl, twh, kc);
+   forward_dif<PH, LD, 64, 64, KEEP_F>(r, S + cc * SH, cl, twh, kc);
    // mid: column-spectrum slot cl*8 + k of column cc is 2D slot (cl*8 + k, cc)
    if constexpr(Op::reads_filter) {
       const uint32_t fi = modulo_count(t, p.fcount);
@@ -319,6 +345,8 @@ small2d_kernel(const Small2dParams p)
          // direct reads take 1-4 cache lines per instruction (32 x 32 298 ->
          // 278, 8 x 512 277 -> 258), so those read in place.
          const uint32_t pt0 = (wv * 512u) % (H * W);
+         // x mod SH for x < 2 * SH (here W <= 64 < SH)
+         auto wrap = [](uint32_t x) { return x - SH < x ? x - SH : x; };
          float2 v[8];
 #pragma unroll
          for(int q = 0; q < 8; q++) v[q] = fb.ld2((pt0 + wl) * 8u, q * 512);
@@ -326,11 +354,11 @@ small2d_kernel(const Small2dParams p)
 #pragma unroll
          for(int q = 0; q < 8; q++) {
             const uint32_t pt = pt0 + q * 64 + wl, row = pt / W, col = pt % W;
-            S[col * SH + (row + row / 8 + col) % SH] = v[q];
+            S[col * SH + wrap(row + row / 8 + col)] = v[q];
          }
          __syncthreads();
 #pragma unroll
-         for(int k = 0; k < 8; k++) b[k] = S[cc * SH + (cl * 9 + k + cc) % SH];
+         for(int k = 0; k < 8; k++) b[k] = S[cc * SH + wrap(cl * 9 + k + cc)];
       } else {
 #pragma unroll
          for(int k = 0; k < 8; k++) b[k] = fb.ld2((uint32_t)(cl * 8 * W + cc) * 8u, k * W * 8);
@@ -341,15 +369,22 @@ small2d_kernel(const Small2dParams p)
 #pragma unroll
       for(int k = 0; k < 8; k++) r[k] = Op::apply(r[k], make_float2(0.f, 0.f));
    }
-   inverse_dit<PH, LD, 64, 64, KEEP_USE>(r, S + cc * SH, cl, twh, kc);
-   // transposed back: column cc's rows cl + q*TH to S[cc*CT + row]
-   __syncthreads();
+   inverse_dit<PH, LD, 64, 64, KEEP_I>(r, S + cc * SH, cl, twh, kc);
+   // transposed back; where holding the first crossing's addresses would cost a
+   // wavefront per SIMD, the lane's index is hidden from here on (an empty asm),
+   // so that they are worked out again (4 to 14 VGPRs less: 64 x 128 and 512 x 16
+   // fit 64, two workgroups per CU where there was one)
+   constexpr bool AGAIN = TN::bits >= 2 || H * W > 4096 || (W == 8 && H >= 128);
+   int j = i;
+   if constexpr(AGAIN) asm volatile("" : "+v"(j));
+   const int rr2 = j / TW, rl2 = j % TW, cc2 = j / TH, cl2 = j % TH;
+   pass_barrier<64>();
 #pragma unroll
-   for(int q = 0; q < 8; q++) S[cc * CT + cl + q * TH] = r[q];
+   for(int q = 0; q < 8; q++) S[TN::slot(cc2, cl2 + q * TH)] = r[q];
    __syncthreads();
    // rows DIT: lane (rr, rl) takes row rr's spectrum slots rl*8 + k
 #pragma unroll
-   for(int k = 0; k < 8; k++) r[k] = S[(rl * 8 + k) * CT + rr];
+   for(int k = 0; k < 8; k++) r[k] = S[TN::slot(rl2 * 8 + k, rr2)];
    __syncthreads();
    inverse_dit<PW, LD, 64>(r, S + rr * SW, rl, tww);
    if constexpr(STAGE) {

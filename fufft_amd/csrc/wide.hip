@@ -174,19 +174,22 @@ __device__ __forceinline__ void wide_mid(float2 (&r)[PL::V], const Buf& fb, uint
 {
    using Op = MidOf<MID>;
    constexpr int T = PL::T, G = 2, T16 = PL::N / 16;
+   // slots whose loads are in flight: four; at N = 16384 digit order fits 128
+   // VGPRs with two, bperm with eight
+   constexpr int FLY = PL::N != 16384 || FLT == FLT_LANE ? 4 : FLT == FLT_BPERM ? 8 : 2;
 #pragma unroll
    for(int g = 0; g < G; g++) {
       const uint32_t l16 = (uint32_t)(L + g * T);
-      // at most 4 slots' loads in flight (the empty asm orders each step after
+      // at most FLY slots' loads in flight (the empty asm orders each step after
       // the last): all 16 at once pushed the kernel past 128 VGPRs into scratch
       if constexpr(FLT == FLT_BPERM) {
 #pragma unroll
-         for(int h = 0; h < 16; h += 4) {
-            float2 f[4];
+         for(int h = 0; h < 16; h += FLY) {
+            float2 f[FLY];
 #pragma unroll
-            for(int k = 0; k < 4; k++) f[k] = fb.ld2((fb0 + l16) * 8u, (h + k) * T16 * 8);
+            for(int k = 0; k < FLY; k++) f[k] = fb.ld2((fb0 + l16) * 8u, (h + k) * T16 * 8);
 #pragma unroll
-            for(int k = 0; k < 4; k++) {
+            for(int k = 0; k < FLY; k++) {
                r[g + G * (h + k)] = Op::apply(r[g + G * (h + k)], f[k]);
                asm volatile("" :: "v"(r[g + G * (h + k)].x));
             }
@@ -196,12 +199,12 @@ __device__ __forceinline__ void wide_mid(float2 (&r)[PL::V], const Buf& fb, uint
          const uint32_t so = lane ? fb0 * 8u + l16 * 16u : (fb0 + l16 * 16u) * 8u;
          constexpr uint32_t ms = lane ? (uint32_t)T16 * 16u : 16u;
 #pragma unroll
-         for(int h = 0; h < 8; h += 2) {
-            float4 q[2];
+         for(int h = 0; h < 8; h += FLY / 2) {
+            float4 q[FLY / 2];
 #pragma unroll
-            for(int m = 0; m < 2; m++) q[m] = fb.ld4(so, (h + m) * ms);
+            for(int m = 0; m < FLY / 2; m++) q[m] = fb.ld4(so, (h + m) * ms);
 #pragma unroll
-            for(int m = 0; m < 2; m++) {
+            for(int m = 0; m < FLY / 2; m++) {
                const int a = g + G * (2 * (h + m)), b = g + G * (2 * (h + m) + 1);
                r[a] = Op::apply(r[a], make_float2(q[m].x, q[m].y));
                r[b] = Op::apply(r[b], make_float2(q[m].z, q[m].w));

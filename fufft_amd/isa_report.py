@@ -42,7 +42,8 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 
 KINDS = {0: "conv", 1: "conv_r2", 2: "fwd", 3: "apply", 4: "fwd_r2", 5: "apply_r2",
          6: "c2c_fwd", 7: "c2c_inv", 8: "plan_taps", 9: "conv_timed", 10: "conv_mid",
-         11: "conv_psf", 12: "conv_psf_dr"}
+         11: "conv_psf", 12: "conv_psf_dr", 13: "conv_chain", 14: "conv_near", 15: "apply_rows",
+         16: "c2c_fwd_nt", 17: "c2c_inv_nt"}
 MIDS = {0: "mul", 1: "conj", 2: "none"}
 LAYOUTS = {0: "xor", 1: "pad", 2: "xchg"}
 FILTERS = {0: "dr", 1: "lane", 2: "bperm"}
@@ -149,11 +150,12 @@ def decode_name(name: str) -> dict | None:
         # big: blocks of more than 64 points (LDS rendezvous of the block maxima)
         return {"family": "bfp", "n": n, "v": v, "layout": LAYOUTS[lay],
                 "kind": "conv_blocks" if big else "conv", "mid": MIDS[mid]}
-    # the N = 16384 / 32768 conv (wide.hip): 32 values per lane, float exchanges
-    m = re.search(r"conv_wide_kernelILi(\d+)ELi(\d+)ELi(\d+)E", name)
+    # the N = 16384 / 32768 conv (wide.hip): 32 values per lane, float exchanges;
+    # "wide_chain": the four-step chain's pass order
+    m = re.search(r"conv_wide_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb([01])E", name)
     if m:
-        n, mid, flt = map(int, m.groups())
-        return {"family": "wide", "n": n, "v": 32, "layout": "split", "kind": "conv", "mid": MIDS[mid],
+        n, mid, flt, chain = map(int, m.groups())
+        return {"family": "wide_chain" if chain else "wide", "n": n, "v": 32, "layout": "split", "kind": "conv", "mid": MIDS[mid],
                 "filter": FILTERS[flt]}
     return None
 
@@ -180,10 +182,11 @@ def load(objs=None) -> list:
 DFT_OPS = {2: 4, 4: 16, 8: 56, 16: 168}
 
 
-def plan(n: int, v: int) -> list:
-    """(radix, stride) per DIF pass: leftover radix first, then radix v."""
-    m, lv = n.bit_length() - 1, v.bit_length() - 1
-    rads = ([1 << (m % lv)] if m % lv else []) + [v] * (m // lv)
+def plan(n: int, v: int, chain: bool = False) -> list:
+    """(radix, stride) per DIF pass: leftover radix first, then radix v; chain:
+    a radix-16 pass before the plan of n / 16 (the four-step chain)."""
+    m, lv = n.bit_length() - 1 - (4 if chain else 0), v.bit_length() - 1
+    rads = ([16] if chain else []) + ([1 << (m % lv)] if m % lv else []) + [v] * (m // lv)
     out, M = [], n
     for r in rads:
         M //= r
@@ -191,15 +194,32 @@ def plan(n: int, v: int) -> list:
     return out
 
 
+def pass_ops(v: int, r: int, stride: int, lanes: int) -> int:
+    """fp32 operations per lane of one pass of radix r: v / r butterflies and, at
+    stride > 1, the twiddle products, (r - 1) applied per group and (r - 2)
+    generated per chain; the groups share one chain where stride <= lanes."""
+    g = v // r
+    ops = g * DFT_OPS[r]
+    if stride > 1:
+        ops += 4 * ((r - 1) * g + (r - 2) * (1 if stride <= lanes else g))
+    return ops
+
+
 def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
     """Per-lane fp32 arithmetic and LDS accesses, per-wavefront vector-memory
     instructions, of one kernel (digit-order filter)."""
-    if kind == "conv_mid":               # the four-step middle: the conv with another cache policy
+    if kind in ("conv_mid", "conv_near"):   # the conv with another cache policy
         kind = "conv"
-    ps = plan(n, v)
-    one_dir =sum((v // r) * (DFT_OPS[r] + (4 * (2 * r - 3) if M > 1 else 0)) for r, M in ps)
+    kind = kind.removesuffix("_nt")
+    chain = kind == "conv_chain"            # read as the digit-order conv, without its other filter layout
+    if chain:
+        kind = "conv"
+    if kind == "apply_rows":
+        kind, mid = "apply_r2", "none"
+    ps = plan(n, v, chain)
+    one_dir = sum(pass_ops(v, r, M, n // v) for r, M in ps)
     exchanges = len(ps) - 1
-    twiddle_slots = sum(v // r for r, M in ps if M > 1)
+    twiddle_slots = sum(1 if M <= n // v else v // r for r, M in ps if M > 1)
     two = kind in ("conv", "conv_r2", "conv_timed", "conv_psf", "conv_psf_dr")
     arith = one_dir * (2 if two else 1)
     # the forward's last twiddled pass hands its chain to the inverse when that
@@ -236,26 +256,24 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
     # digit-order and pair spectrum stores take one code path (the offsets are selected); a
     # bperm filter read has kernels of its own (conv1d_bperm_kernel, bfp_bperm_kernel).
     untaken_loads = v // 2 if (kind in ("conv", "conv_r2", "conv_timed", "apply", "apply_r2") and mid != "none") else 0
-    if kind in ("apply", "apply_r2"):
-        untaken_loads += v // 2
     untaken = {"loads": untaken_loads, "stores": v if kind == "plan_taps" else 0}
     return {"fp32_arith_per_lane": arith, "lds_access_8B_per_lane": lds, "vmem_loads_per_wave": loads,
             "vmem_stores_per_wave": stores, "untaken_branch": untaken, "passes": ps}
 
 
-def model_wide(mid: str = "mul", filt: str = "lane", n: int = 32768, v: int = 32) -> dict:
+def model_wide(mid: str = "mul", filt: str = "lane", n: int = 32768, v: int = 32, chain: bool = False) -> dict:
     """The N = 16384 / 32768 conv (wide.hip): the radix-16 plan with V/R groups
     per lane in every pass (8 / 4 in the radix-4 / radix-8 lead, 2 in the
     radix-16 passes), no kept chain; each exchange writes and reads both float
     components of the lane's V values (V 8-byte equivalents each way); the
     filter as V/2 16-byte loads (V 8-byte ones in bperm).  A lead pass of more
     than 4 groups per lane reads its base twiddles again for the inverse."""
-    ps = plan(n, 16)
-    one_dir = sum((v // r) * (DFT_OPS[r] + (4 * (2 * r - 3) if M > 1 else 0)) for r, M in ps)
+    ps = plan(n, 16, chain)
+    one_dir = sum(pass_ops(v, r, M, n // v) for r, M in ps)
     arith = 2 * one_dir + (4 * v if mid != "none" else 0)
     lds = 2 * v * (len(ps) - 1) * 2
-    # a pass with M <= T gives both of a lane's groups the same base twiddle
-    # index ((L + g T) mod M = L mod M), and the compiler merges those loads
+    # a pass with M <= T gives all of a lane's groups the same base twiddle
+    # index ((L + g T) mod M = L mod M): one load
     t = n // v
     loads = v + sum((v // r) if M > t else 1 for r, M in ps if M > 1)
     if v // ps[0][0] > 4:
@@ -284,7 +302,7 @@ def default_layout(n: int, v: int, family: str = "conv1d") -> str:
     plan (bfp_lds_layout in bfp.hip)."""
     if family == "bfp":
         return "xchg"
-    if family == "wide":
+    if family in ("wide", "wide_chain"):
         return "split"
     return "pad" if (v == 8 and n > 4096) else "xchg"
 
@@ -306,10 +324,11 @@ def conv_rows(rows=None) -> list:
         t = n // v
         threads = t if t >= 128 else 256
         # the wide kernel's float buffer: N + N/16 slots of 4 bytes
-        lds = (n + n // 16) * 4 if d["family"] == "wide" else lds_bytes_conv(n, v, d["layout"])
+        wide = d["family"] in ("wide", "wide_chain")
+        lds = (n + n // 16) * 4 if wide else lds_bytes_conv(n, v, d["layout"])
         occ = occupancy(r["meta"]["vgpr_count"], r["meta"].get("agpr_count", 0), lds, threads // 64)
         mod = model_conv(n, v, d["kind"], d["mid"]) if d["family"] == "conv1d" else \
-            model_wide(d["mid"], d["filter"], n) if d["family"] == "wide" else None
+            model_wide(d["mid"], d["filter"], n, chain=d["family"] == "wide_chain") if wide else None
         out.append({**d, "vgpr": r["meta"]["vgpr_count"], "sgpr": r["meta"]["sgpr_count"],
                     "scratch": r["meta"].get("private_segment_fixed_size", 0),
                     "spills": r["meta"].get("vgpr_spill_count", 0) + r["meta"].get("sgpr_spill_count", 0),
@@ -344,7 +363,7 @@ def main() -> None:
         vm = (f"{r['vmem_load']}+{r['vmem_store']} / {m['vmem_loads_per_wave'] + m['untaken_branch']['loads']}"
               f"+{m['vmem_stores_per_wave'] + m['untaken_branch']['stores']}") if m else \
             f"{r['vmem_load']}+{r['vmem_store']} / —"
-        label = f"{r['family']} {r['kind']}" + (f" ({r['filter']} filter)" if r["family"] == "wide" else "")
+        label = f"{r['family']} {r['kind']}" + (f" ({r['filter']} filter)" if "filter" in r else "")
         print(f"| {label} | {r['n']} | {r['v']} | {r['vgpr']} | {r['scratch']} | "
               f"{r['waves_per_simd']} ({r['limited_by']}) | {r['valu']} | {ar} | {ld} | {vm} |")
 

@@ -576,6 +576,7 @@ int fufft_conv_f32(const void* in, const void* filt, int64_t filt_stride,
    const int kind = per_signal && layout == FUFFT_LAYOUT_LANE &&
                     (conv_psf_plan((int)n, v) || conv_psf_late_plan((int)n, v))             ? K_CONV_PSF
                   : per_signal && layout == FUFFT_LAYOUT_DR && conv_psf_dr_plan((int)n, v) ? K_CONV_PSF_DR
+                  : conv_near(n, batch) && lds_layout() != LAYOUT_XOR                      ? K_CONV_NEAR
                                                                                            : K_CONV;
    return run_conv1d(kind, (int)n, v, p, stream);
 }
@@ -697,7 +698,9 @@ int fufft_c2c_f32(const void* in, void* out, int64_t n, int64_t batch, int direc
    if((st = current_table(&p.tw)) != FUFFT_OK) return st;
    p.in0 = in; p.out0 = out; p.ntrans = (uint32_t)batch;
    p.fcount = 1; p.scount = 1; p.mid = FUFFT_MID_NONE; p.fl = FUFFT_LAYOUT_DR;
-   return run_conv1d(direction == FUFFT_FORWARD ? K_C2C_FWD : K_C2C_INV, (int)n, v, p, stream);
+   const bool nt = c2c_streams(n, batch);
+   const int kind = direction == FUFFT_FORWARD ? (nt ? K_C2C_FWD_NT : K_C2C_FWD) : (nt ? K_C2C_INV_NT : K_C2C_INV);
+   return run_conv1d(kind, (int)n, v, p, stream);
 }
 
 // ---- filter planning on the device -------------------------------------------------------
@@ -1419,7 +1422,7 @@ int fufft_conv2d_f32(const void* in, const void* filt, int64_t filt_stride, void
       if(e != hipSuccess) return status_of(e);
       r = rows_params(tw, h, nb);
       r.spec = dst; r.scount = r.ntrans; r.out0 = dst;
-      if((st = run_conv1d(K_APPLY, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
+      if((st = run_conv1d(K_APPLY_ROWS, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
    }
    return FUFFT_OK;
 }
@@ -1540,7 +1543,7 @@ int fufft_apply2d_f32(const void* spec, int64_t spec_stride, const void* filt, i
       if(e != hipSuccess) return status_of(e);
       Conv1dParams r = rows_params(tw, h, nb);
       r.spec = dst; r.scount = r.ntrans; r.out0 = dst;
-      if((st = run_conv1d(K_APPLY, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
+      if((st = run_conv1d(K_APPLY_ROWS, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
    }
    return FUFFT_OK;
 }

@@ -90,10 +90,11 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // u / v) travel as two separate float arrays
    constexpr bool REAL_IN   = KIND == K_CONV_R2 || KIND == K_FWD_R2;
    constexpr bool REAL_OUT  = KIND == K_CONV_R2 || KIND == K_APPLY_R2;
-   constexpr bool FROM_SPEC = KIND == K_APPLY || KIND == K_APPLY_R2;
+   constexpr bool FROM_ROWS = KIND == K_APPLY_ROWS || KIND == K_APPLY_R2;   // 2D rows: lane-major spectra
+   constexpr bool FROM_SPEC = KIND == K_APPLY || FROM_ROWS;
    constexpr bool TO_SPEC   = KIND == K_FWD || KIND == K_FWD_R2;
-   constexpr bool C2C_FWD   = KIND == K_C2C_FWD;
-   constexpr bool C2C_INV   = KIND == K_C2C_INV;
+   constexpr bool C2C_FWD   = KIND == K_C2C_FWD || KIND == K_C2C_FWD_NT;
+   constexpr bool C2C_INV   = KIND == K_C2C_INV || KIND == K_C2C_INV_NT;
    constexpr bool PLAN      = KIND == K_PLAN_TAPS;
    constexpr bool TIMED     = KIND == K_CONV_TIMED;
    // one filter per signal: its loads go out with the signal's (lane-major
@@ -104,11 +105,17 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // where the registers allow no early read: the lane-major filter read at
    // the mid as usual, streamed past the caches
    constexpr bool PSF_LATE  = PSF_ANY && !PSF;
-   // the signal read and the result written once per launch stream past the
-   // caches in the single-launch conv and C2C; the four-step middle, the split
-   // and 2D row kernels keep the default policy
-   constexpr int  IO_POL    = (KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED ||
-                               C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
+   // Cache policy of the signal's loads and the result's stores (conv_near in
+   // fufft_internal.hpp has the measurements).  The single-launch kinds write
+   // their result past the caches (NT), which leaves these to what is read;
+   // the loads stream too where the signals are more than the last-level cache
+   // keeps.  The four-step middle, the split forward and the 2D rows hand their
+   // data to the next launch: default both ways.  So does a large C2C, whose
+   // result is the next call's input (c2c_streams in fufft_internal.hpp).
+   constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
+   constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
+   constexpr int  ST_POL = (ONCE || KIND == K_CONV_NEAR || KIND == K_CONV_R2 || KIND == K_APPLY ||
+                             KIND == K_C2C_FWD_NT || KIND == K_C2C_INV_NT) ? POL_NT : POL_DEFAULT;
    constexpr int  EL_IN     = REAL_IN ? 4 : 8;
    constexpr int  EL_OUT    = REAL_OUT ? 4 : 8;
 
@@ -140,7 +147,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    Twiddles<PL> tw;
    tw.load(p.tw, L);
    // both halves in this launch: the forward's last twiddled chain serves the inverse
-   constexpr int KEEP_F = (KIND == K_CONV || KIND == K_CONV_MID || KIND == K_CONV_R2 || TIMED || PSF_LATE) ? KEEP_STORE
+   constexpr int KEEP_F = (KIND == K_CONV || KIND == K_CONV_NEAR || KIND == K_CONV_MID || KIND == K_CONV_R2 || TIMED || PSF_LATE) ? KEEP_STORE
                                                                                                       : KEEP_NONE;
    constexpr int KEEP_I = KEEP_F == KEEP_STORE ? KEEP_USE : KEEP_NONE;
    KeptChain<PL> kc;
@@ -149,7 +156,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
 
    if constexpr(FROM_SPEC) {
       const Buf sb(p.spec, p.scount * (uint32_t)N * 8u);
-      if(p.sl == FLT_LANE) {
+      if constexpr(FROM_ROWS) {
          // lane-major pairs: slots L*V + 2m, 2m + 1 at 2(L + m*T), one
          // contiguous KiB per 16-byte load of a wavefront
          const uint32_t so = modulo_count(t, p.scount) * N * 8u + L * 16u;
@@ -196,11 +203,11 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
          const Buf yb(static_cast<const char*>(p.in1) + wb, WB);
 #pragma unroll
          for(int q = 0; q < V; q++)
-            r[q] = make_float2(xb.ld1(lane_pos * 4u, q * T * 4), yb.ld1(lane_pos * 4u, q * T * 4));
+            r[q] = make_float2(xb.ld1<LD_POL>(lane_pos * 4u, q * T * 4), yb.ld1<LD_POL>(lane_pos * 4u, q * T * 4));
       } else {
          const Buf xb(static_cast<const char*>(p.in0) + wb, WB);
 #pragma unroll
-         for(int q = 0; q < V; q++) r[q] = xb.ld2<IO_POL>(lane_pos * 8u, q * T * 8);
+         for(int q = 0; q < V; q++) r[q] = xb.ld2<LD_POL>(lane_pos * 8u, q * T * 8);
       }
       if constexpr(PSF) {
          // each signal's own filter is a third stream from HBM: issued here,
@@ -231,7 +238,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
       digit_to_natural<PL, LD, LANES>(r, A, L);
       const Buf ob(static_cast<char*>(p.out0) + (size_t)t0 * N * 8, TPW * N * 8);
 #pragma unroll
-      for(int q = 0; q < V; q++) ob.st2<IO_POL>(r[q], lane_pos * 8u, q * T * 8);
+      for(int q = 0; q < V; q++) ob.st2<ST_POL>(r[q], lane_pos * 8u, q * T * 8);
       return;
    } else if constexpr(PLAN) {
       const Buf ob(static_cast<char*>(p.out0) + (size_t)t0 * N * 8, TPW * N * 8);
@@ -296,13 +303,13 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
          const Buf vb(static_cast<char*>(p.out1) + wb, WB);
 #pragma unroll
          for(int q = 0; q < V; q++) {
-            ub.st1(r[q].x, lane_pos * 4u, q * T * 4);
-            vb.st1(r[q].y, lane_pos * 4u, q * T * 4);
+            ub.st1<ST_POL>(r[q].x, lane_pos * 4u, q * T * 4);
+            vb.st1<ST_POL>(r[q].y, lane_pos * 4u, q * T * 4);
          }
       } else {
          const Buf ob(static_cast<char*>(p.out0) + wb, WB);
 #pragma unroll
-         for(int q = 0; q < V; q++) ob.st2<IO_POL>(r[q], lane_pos * 8u, q * T * 8);
+         for(int q = 0; q < V; q++) ob.st2<ST_POL>(r[q], lane_pos * 8u, q * T * 8);
       }
       if constexpr(TIMED) {
          stamp(5);
@@ -358,7 +365,7 @@ template<int LAYOUT, int KIND, int MID>
 constexpr bool reads_bperm_filter()
 {
    return LAYOUT != LAYOUT_XOR && mid_reads_filter<MID> &&
-          (KIND == K_CONV || KIND == K_CONV_TIMED || KIND == K_CONV_R2 || KIND == K_APPLY);
+          (KIND == K_CONV || KIND == K_CONV_NEAR || KIND == K_CONV_TIMED || KIND == K_CONV_R2 || KIND == K_APPLY);
 }
 
 template<int N, int V, int LAYOUT, int KIND, int MID>
@@ -398,6 +405,9 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
 {
    switch(kind) {
       case K_CONV:    return launch_mid<N, V, LAYOUT, K_CONV>(p, s);
+      case K_CONV_NEAR:
+         if constexpr(conv_near_plan(N) && LAYOUT != LAYOUT_XOR) return launch_mid<N, V, LAYOUT, K_CONV_NEAR>(p, s);
+         else                                                    return hipErrorInvalidValue;
       case K_CONV_PSF:
          // lane-major filters only, default LDS layouts (the launcher's choice)
          if constexpr((conv_psf_plan(N, V) || conv_psf_late_plan(N, V)) && LAYOUT != LAYOUT_XOR) {
@@ -427,6 +437,9 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
       case K_CONV_R2: return launch_one<N, V, LAYOUT, K_CONV_R2, MID_MUL>(p, s);
       case K_FWD:     return launch_one<N, V, LAYOUT, K_FWD, MID_NONE>(p, s);
       case K_APPLY:   return launch_mid<N, V, LAYOUT, K_APPLY>(p, s);
+      case K_APPLY_ROWS:
+         // the row inverse of the 2D paths
+         return p.mid == MID_NONE ? launch_one<N, V, LAYOUT, K_APPLY_ROWS, MID_NONE>(p, s) : hipErrorInvalidValue;
       case K_FWD_R2:  return launch_one<N, V, LAYOUT, K_FWD_R2, MID_NONE>(p, s);
       case K_APPLY_R2:
          // only the 2D two-for-one path uses it, as the row inverse
@@ -434,6 +447,8 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
                                   : hipErrorInvalidValue;
       case K_C2C_FWD:   return launch_one<N, V, LAYOUT, K_C2C_FWD, MID_NONE>(p, s);
       case K_C2C_INV:   return launch_one<N, V, LAYOUT, K_C2C_INV, MID_NONE>(p, s);
+      case K_C2C_FWD_NT: return launch_one<N, V, LAYOUT, K_C2C_FWD_NT, MID_NONE>(p, s);
+      case K_C2C_INV_NT: return launch_one<N, V, LAYOUT, K_C2C_INV_NT, MID_NONE>(p, s);
       case K_PLAN_TAPS: return launch_one<N, V, LAYOUT, K_PLAN_TAPS, MID_NONE>(p, s);
       case K_CONV_TIMED:
          // the timed build exists for the default LDS layout only

@@ -393,11 +393,11 @@ small2d_kernel(const Small2dParams p)
       pass_barrier<64>();
       const Buf wb(static_cast<char*>(p.out) + wp * 8u, wbytes);
 #pragma unroll
-      for(int q = 0; q < 8; q++) wb.st2(lds[stage_slot(q * 64 + wl)], wl * 8u, q * 512);
+      for(int q = 0; q < 8; q++) wb.st2<POL_NT>(lds[stage_slot(q * 64 + wl)], wl * 8u, q * 512);
    } else {
       const Buf ob(static_cast<char*>(p.out) + (size_t)t * BYTES, live ? BYTES : 0u);
 #pragma unroll
-      for(int q = 0; q < 8; q++) ob.st2(r[q], (uint32_t)(rr * W + rl) * 8u, q * TW * 8);
+      for(int q = 0; q < 8; q++) ob.st2<POL_NT>(r[q], (uint32_t)(rr * W + rl) * 8u, q * TW * 8);
    }
 }
 

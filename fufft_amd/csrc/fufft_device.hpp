@@ -284,9 +284,10 @@ struct Buf {
    __device__ __forceinline__ Buf(const void* base, uint32_t bytes)
       : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, kFlags)) {}
 
+   template<int POL = POL_DEFAULT>
    __device__ __forceinline__ float ld1(uint32_t voff, uint32_t soff) const
    {
-      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, POL));
    }
    template<int POL = POL_DEFAULT>
    __device__ __forceinline__ float2 ld2(uint32_t voff, uint32_t soff) const
@@ -307,9 +308,10 @@ struct Buf {
    {
       return (int)(int8_t)__builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0);
    }
+   template<int POL = POL_DEFAULT>
    __device__ __forceinline__ void st1(float v, uint32_t voff, uint32_t soff) const
    {
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, POL);
    }
    template<int POL = POL_DEFAULT>
    __device__ __forceinline__ void st2(float2 v, uint32_t voff, uint32_t soff) const

@@ -43,6 +43,10 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 }
 
 // ---- 1D fused pipeline (conv1d.hip) ------------------------------------------------
+// K_APPLY: the split apply, spectra in digit order; K_APPLY_ROWS: the row
+// inverse of the 2D paths, lane-major spectra and no mid operation.
+// K_CONV_NEAR: K_CONV for signals that the last-level cache keeps: default
+// loads (conv_near).
 // K_FWD_R2 / K_APPLY_R2: the forward half reading two real arrays, the
 // inverse half writing two real arrays (2D two-for-one rows).
 // K_C2C_FWD / K_C2C_INV: natural order in and out (forward DIF + digit ->
@@ -66,7 +70,8 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 // through LDS at the mid operation.
 enum { K_CONV = 0, K_CONV_R2 = 1, K_FWD = 2, K_APPLY = 3, K_FWD_R2 = 4, K_APPLY_R2 = 5,
        K_C2C_FWD = 6, K_C2C_INV = 7, K_PLAN_TAPS = 8, K_CONV_TIMED = 9, K_CONV_MID = 10,
-       K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13 };
+       K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13,
+       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_C2C_FWD_NT = 16, K_C2C_INV_NT = 17 };
 
 // the plans K_CONV_PSF and K_CONV_PSF_DR are built for: radix 16 with whole
 // wavefronts per transform and room for the filter's 32 VGPRs within 128
@@ -86,6 +91,40 @@ constexpr bool conv_psf_dr_plan(int n, int v) { return v == 16 && (n == 2048 || 
 // 213.3, so those sizes keep the plain kernel.
 constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 
+// K_CONV_NEAR runs the conv whose signals take under half of the 256 MiB
+// last-level cache.  What a program convolves was mostly just written, or is
+// convolved again, and a default load keeps it there, where a streaming one
+// has the next pass fetch it from HBM.  Three states in turn, us, loads and
+// stores streamed / only the stores / neither:
+//   N = 1024, digit order: 2 M points 8.8 / 8.9 / 10.8, 6 M 22.8 / 19.0 / 24.4, 8 M
+//     29.3 / 23.8 / 29.9, 10 M 35.2 / 29.2 / 37.4, 17 M (128 MiB) 53.1 / 54.3 / 54.7, 67 M
+//     195.8 / 197.4 / 200.2;
+//   N = 512: 8 M 26.0 / 21.7 / 27.7; N = 4096: 8 M 29.8 / 26.1 / 30.0; N = 8192: 8 M
+//     38.1 / 36.2 / 40.6; N = 16384 and 32768 even.
+// The other single-launch kinds have one policy.  Stores streamed, loads not:
+// the split apply (N = 512 / 4096 / 8192, 8 M points 29.3 / 33.6 / 38.9 -> 24.3 / 26.9
+// / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv (8 M, N = 256 / 4096 30.9 /
+// 31.9 -> 26.0 / 26.5) and the small images; both streamed: one filter per signal,
+// the four-step chain and N >= 16384, which measured best or even so.
+constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
+constexpr bool conv_near(int64_t n, int64_t batch)
+{
+   return conv_near_plan(n) && batch < ((int64_t)128 << 20) / (8 * n);
+}
+
+// A C2C's result is the next call's input (a spectrum on its way back), so it is
+// stored where that call finds it, unless the L2s (32 MiB together) would hold
+// it all, whose lines the end of the kernel then has to write back, or it is
+// more than the 256 MiB last-level cache.  Forward and inverse, us, stores
+// streamed / not: N = 4096, 16 MiB 15.6 / 18.2, 32 MiB 29.6 / 26.5, 48 MiB 42.4 /
+// 36.2, 256 MiB 174.9 / 166.9, 320 MiB 217 / 230, 512 MiB 350 / 365; N = 512, 16 MiB
+// 14.6 / 15.5, 48 MiB 37.3 / 33.9, 256 MiB 171.3 / 164.7, 384 MiB 253 / 259.
+constexpr bool c2c_streams(int64_t n, int64_t batch)
+{
+   const int64_t mib32 = ((int64_t)32 << 20) / (8 * n);      // transforms in 32 MiB
+   return batch < mib32 || batch > 8 * mib32;
+}
+
 // phase timer record of one workgroup (K_CONV_TIMED), TIMER_STRIDE words:
 // [0] HW_ID, [1] XCC_ID, [2] marks, [3] s_memrealtime ticks (100 MHz) from
 // the first mark to the last, [4..5] start (s_memtime, lo / hi),
@@ -96,7 +135,7 @@ enum { TIMER_STRIDE = 12, TIMER_MARKS = 5 };
 struct Conv1dParams {
    const void*   in0;      // complex input, or real x (K_CONV_R2)
    const void*   in1;      // real y (K_CONV_R2)
-   const void*   spec;     // spectrum (K_APPLY), laid out as sl says
+   const void*   spec;     // spectrum (K_APPLY digit order, the row inverses lane-major)
    const void*   filt;     // filter, digit order or lane-major
    void*         out0;     // complex output / spectrum (K_FWD) / real u
    void*         out1;     // real v (K_CONV_R2)
@@ -106,7 +145,7 @@ struct Conv1dParams {
    uint32_t      scount;   // transform t uses spectrum (t % scount)
    int32_t       mid;      // a registered mid policy id (FUFFT_MID_POLICIES)
    int32_t       fl;       // FLT_DR / FLT_LANE (filter read; K_PLAN_TAPS: layout written)
-   int32_t       sl;       // FLT_DR / FLT_LANE: spectrum K_FWD writes, K_APPLY reads
+   int32_t       sl;       // FLT_DR / FLT_LANE: spectrum K_FWD writes
    float         scale;    // K_PLAN_TAPS: factor applied to the spectrum
    uint32_t*     timing;   // K_CONV_TIMED: TIMER_STRIDE words per workgroup
    uint32_t      timing_groups;   // workgroups that write a record

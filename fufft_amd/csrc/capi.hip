@@ -698,9 +698,7 @@ int fufft_c2c_f32(const void* in, void* out, int64_t n, int64_t batch, int direc
    if((st = current_table(&p.tw)) != FUFFT_OK) return st;
    p.in0 = in; p.out0 = out; p.ntrans = (uint32_t)batch;
    p.fcount = 1; p.scount = 1; p.mid = FUFFT_MID_NONE; p.fl = FUFFT_LAYOUT_DR;
-   const bool nt = c2c_streams(n, batch);
-   const int kind = direction == FUFFT_FORWARD ? (nt ? K_C2C_FWD_NT : K_C2C_FWD) : (nt ? K_C2C_INV_NT : K_C2C_INV);
-   return run_conv1d(kind, (int)n, v, p, stream);
+   return run_conv1d(direction == FUFFT_FORWARD ? K_C2C_FWD : K_C2C_INV, (int)n, v, p, stream);
 }
 
 // ---- filter planning on the device -------------------------------------------------------
@@ -1065,25 +1063,25 @@ int fufft_plan_filter_large_device_f32(const void* in, void* out, int64_t n, int
 // How many of a batch's four-step transforms run the whole chain in one
 // workgroup each (radix-16 middle, n <= 32768), reading and writing the data
 // once where the three launches do it three times; the rest run those.  The
-// results are the same bit for bit, so the line is the faster side.  us a call,
-// shared filter, four buffers in turn, three launches / one:
-//   n =  8192: batch 1 12.7 / 9.8, 64 14.5 / 10.5, 256 23.6 / 12.7, 4096 241 / 124;
-//   n = 16384: 24 14.1 / 15.4, 48 17.0 / 16.4, 64 19.2 / 16.6, 128 25.4 / 17.6, 4096
-//     490 / 299;
-//   n = 32768: 80 34.4 / 35.5, 100 36.0 / 36.1, 128 39.4 / 38.4, 192 55.3 / 42.6,
-//     256 70.5 / 55.7, 512 131 / 107, 768 189 / 158, 4096 975 / 674.
-// At n = 32768 a transform fills a CU for some 32 us, so a last round of under
-// 100 of them is left to the three launches (530: 135 / 137, so 125), and one
-// full round with 32 or more behind it is not worth splitting (301: 81.3 / 87.9,
-// split 82.4).
+// results are the same bit for bit, so the line is the faster side.  A round of
+// up to 256 transforms (one per CU, where it holds no more) takes some 17 us at
+// n = 16384 and 35 at 32768, full or not, so a last round of a few is left to the
+// three launches.  us a call, shared filter, three buffers in turn, three launches
+// / one / split (whole rounds in one):
+//   n =  8192: 1 11.6 / 9.5, 64 12.4 / 10.1, 200 18.0 / 12.5, 400 32.8 / 18.6;
+//   n = 16384: 40 12.8 / 16.4, 64 14.8 / 16.7, 80 16.9 / 16.8, 128 20.2 / 17.5, 256
+//     36.6 / 21.8, 300 41.6 / 36.0 / 34.0, 340 47.2 / 37.3 / 38.3, 512 65.0 / 49.6;
+//   n = 32768: 100 29.2 / 35.6, 128 33.9 / 38.4, 160 42.9 / 40.8, 256 62.5 / 52.1, 301
+//     72.8 / 84.7 / 69.1, 384 92.5 / 88.9 / 86.2, 448 107 / 93 / 101, 530 125 / 132 /
+//     113, 768 181 / 149.
+// A filter per transform moves the lines little (n = 32768: 128 37.0 / 39.9, 160 46.7 /
+// 44.4, 384 109 / 95 / 94).
 static int64_t chain_batch(int64_t n, int v, int64_t batch)
 {
    if(!conv_chain_plan(n, v)) return 0;
    if(n == 8192) return batch;
-   if(n == 16384) return batch >= 48 ? batch : 0;
    const int64_t last = batch % 256;
-   if(last >= 100) return batch;
-   return batch < 512 && last >= 32 ? 0 : batch - last;
+   return last >= (n == 16384 ? 80 : 144) ? batch : batch - last;
 }
 
 int fufft_conv_large_f32(void* buf, const void* filt, int64_t filt_stride, int64_t n,
@@ -1216,7 +1214,6 @@ Conv1dParams rows_params(const float2* tw, int64_t h, int64_t batch)
    p.tw = tw;
    p.ntrans = (uint32_t)(h * batch);
    p.fcount = 1; p.scount = 1; p.mid = FUFFT_MID_NONE; p.fl = FUFFT_LAYOUT_DR;
-   p.sl = FUFFT_LAYOUT_LANE;
    return p;
 }
 
@@ -1412,7 +1409,7 @@ int fufft_conv2d_f32(const void* in, const void* filt, int64_t filt_stride, void
       // rows DIT in place
       Conv1dParams r = rows_params(tw, h, nb);
       r.in0 = src; r.out0 = dst;
-      if((st = run_conv1d(K_FWD, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
+      if((st = run_conv1d(K_FWD_ROWS, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
       ColParams c = col_params(tw, w, nb);
       set_filter_layout(c, pl, w, layout);
       c.in = dst; c.out = dst; c.mid = mid;
@@ -1495,7 +1492,7 @@ int fufft_fwd2d_f32(const void* in, void* spec, int64_t h, int64_t w, int64_t ba
       char* dst = static_cast<char*>(spec) + i0 * np * 8;
       Conv1dParams r = rows_params(tw, h, nb);
       r.in0 = static_cast<const char*>(in) + i0 * np * 8; r.out0 = dst;
-      if((st = run_conv1d(K_FWD, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
+      if((st = run_conv1d(K_FWD_ROWS, (int)w, pl.vr, r, stream)) != FUFFT_OK) return st;
       ColParams c = col_params(tw, w, nb);
       c.in = dst; c.out = dst;
       const hipError_t e = launch_col(COL_FWD, (int)h, c, static_cast<hipStream_t>(stream));

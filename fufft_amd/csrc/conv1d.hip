@@ -61,7 +61,7 @@ inline uint32_t conv_iters(uint32_t ntrans)
 // offset base) as 16-byte pairs: contiguous in digit order, at 2(L + m*T)
 // lane-major (FLT_LANE).  One uniform branch; each side computes only its own
 // offsets.
-template<int V, int T>
+template<int V, int T, int POL>
 __device__ __forceinline__ void store_spectrum(const Buf& ob, const float2 (&r)[V], uint32_t base, int L, int layout)
 {
    const bool lane = layout == FLT_LANE;
@@ -69,7 +69,7 @@ __device__ __forceinline__ void store_spectrum(const Buf& ob, const float2 (&r)[
    const uint32_t ms = lane ? (uint32_t)T * 16u : 16u;
 #pragma unroll
    for(int m = 0; m < V / 2; m++)
-      ob.st4(make_float4(r[2 * m].x, r[2 * m].y, r[2 * m + 1].x, r[2 * m + 1].y), so, m * ms);
+      ob.st4<POL>(make_float4(r[2 * m].x, r[2 * m].y, r[2 * m + 1].x, r[2 * m + 1].y), so, m * ms);
 }
 
 // The kernel body for transform group bid.  BPERM: the filter is in the
@@ -92,9 +92,9 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    constexpr bool REAL_OUT  = KIND == K_CONV_R2 || KIND == K_APPLY_R2;
    constexpr bool FROM_ROWS = KIND == K_APPLY_ROWS || KIND == K_APPLY_R2;   // 2D rows: lane-major spectra
    constexpr bool FROM_SPEC = KIND == K_APPLY || FROM_ROWS;
-   constexpr bool TO_SPEC   = KIND == K_FWD || KIND == K_FWD_R2;
-   constexpr bool C2C_FWD   = KIND == K_C2C_FWD || KIND == K_C2C_FWD_NT;
-   constexpr bool C2C_INV   = KIND == K_C2C_INV || KIND == K_C2C_INV_NT;
+   constexpr bool TO_SPEC   = KIND == K_FWD || KIND == K_FWD_ROWS || KIND == K_FWD_R2;
+   constexpr bool C2C_FWD   = KIND == K_C2C_FWD;
+   constexpr bool C2C_INV   = KIND == K_C2C_INV;
    constexpr bool PLAN      = KIND == K_PLAN_TAPS;
    constexpr bool TIMED     = KIND == K_CONV_TIMED;
    // one filter per signal: its loads go out with the signal's (lane-major
@@ -105,17 +105,21 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // where the registers allow no early read: the lane-major filter read at
    // the mid as usual, streamed past the caches
    constexpr bool PSF_LATE  = PSF_ANY && !PSF;
-   // Cache policy of the signal's loads and the result's stores (conv_near in
-   // fufft_internal.hpp has the measurements).  The single-launch kinds write
-   // their result past the caches (NT), which leaves these to what is read;
-   // the loads stream too where the signals are more than the last-level cache
-   // keeps.  The four-step middle, the split forward and the 2D rows hand their
-   // data to the next launch: default both ways.  So does a large C2C, whose
-   // result is the next call's input (c2c_streams in fufft_internal.hpp).
+   // Cache policy of the signal's loads and the result's stores (figures at
+   // POL_WT in fufft_device.hpp and conv_near in fufft_internal.hpp).  What the
+   // program's or the path's next launch reads -- 2D rows, the four-step middle,
+   // a C2C spectrum on its way back -- is written through (WT); the other results
+   // stream past the caches (NT), which leaves these to what is read, except at
+   // N = 16384, where writing through measured 2-10% faster (8 M points 52.0 -> 46.4
+   // us).  The loads stream too where the signals are more than the last-level
+   // cache keeps.  The split forward keeps the default: its digit-order stores
+   // are 16-byte pieces that the L2 puts together.
    constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
+   constexpr bool KEPT = KIND == K_CONV_MID || KIND == K_FWD_ROWS || KIND == K_FWD_R2 || KIND == K_APPLY_ROWS ||
+                         KIND == K_APPLY_R2 || C2C_FWD || C2C_INV || (KIND == K_CONV && N == 16384);
    constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
-   constexpr int  ST_POL = (ONCE || KIND == K_CONV_NEAR || KIND == K_CONV_R2 || KIND == K_APPLY ||
-                             KIND == K_C2C_FWD_NT || KIND == K_C2C_INV_NT) ? POL_NT : POL_DEFAULT;
+   constexpr int  ST_POL = KEPT ? POL_WT
+                         : (ONCE || KIND == K_CONV_NEAR || KIND == K_CONV_R2 || KIND == K_APPLY) ? POL_NT : POL_DEFAULT;
    constexpr int  EL_IN     = REAL_IN ? 4 : 8;
    constexpr int  EL_OUT    = REAL_OUT ? 4 : 8;
 
@@ -248,7 +252,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
 #pragma unroll
          for(int k = 0; k < V; k++) ob.st2(r[k], lane_pos * 8u, k * T * 8);
       } else {
-         store_spectrum<V, T>(ob, r, (t - t0) * N, L, p.fl);
+         store_spectrum<V, T, ST_POL>(ob, r, (t - t0) * N, L, p.fl);
       }
       return;
    } else if constexpr(TO_SPEC) {
@@ -256,7 +260,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
       // lane-major: every store of a wavefront is one contiguous run.  The
       // digit-order store writes 16 bytes per lane 64 or 128 bytes apart (32
       // or 64 cache lines per wavefront store) and runs 14-18% slower.
-      store_spectrum<V, T>(ob, r, (t - t0) * N, L, p.sl);
+      store_spectrum<V, T, ST_POL>(ob, r, (t - t0) * N, L, KIND == K_FWD ? FLT_DR : FLT_LANE);
       return;
    } else {
       if constexpr(!C2C_INV) {
@@ -437,6 +441,7 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
       case K_CONV_R2: return launch_one<N, V, LAYOUT, K_CONV_R2, MID_MUL>(p, s);
       case K_FWD:     return launch_one<N, V, LAYOUT, K_FWD, MID_NONE>(p, s);
       case K_APPLY:   return launch_mid<N, V, LAYOUT, K_APPLY>(p, s);
+      case K_FWD_ROWS: return launch_one<N, V, LAYOUT, K_FWD_ROWS, MID_NONE>(p, s);
       case K_APPLY_ROWS:
          // the row inverse of the 2D paths
          return p.mid == MID_NONE ? launch_one<N, V, LAYOUT, K_APPLY_ROWS, MID_NONE>(p, s) : hipErrorInvalidValue;
@@ -447,8 +452,6 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
                                   : hipErrorInvalidValue;
       case K_C2C_FWD:   return launch_one<N, V, LAYOUT, K_C2C_FWD, MID_NONE>(p, s);
       case K_C2C_INV:   return launch_one<N, V, LAYOUT, K_C2C_INV, MID_NONE>(p, s);
-      case K_C2C_FWD_NT: return launch_one<N, V, LAYOUT, K_C2C_FWD_NT, MID_NONE>(p, s);
-      case K_C2C_INV_NT: return launch_one<N, V, LAYOUT, K_C2C_INV_NT, MID_NONE>(p, s);
       case K_PLAN_TAPS: return launch_one<N, V, LAYOUT, K_PLAN_TAPS, MID_NONE>(p, s);
       case K_CONV_TIMED:
          // the timed build exists for the default LDS layout only

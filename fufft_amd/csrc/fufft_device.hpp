@@ -268,13 +268,21 @@ __device__ __forceinline__ void twiddle_group(float2 (&r)[NR], float2 w1)
 // offset, and per-tap offsets ride in the scalar offset field, so a lane keeps
 // one VGPR of addressing instead of a 64-bit pointer per tap.  Accesses beyond
 // num_records bytes read zero and drop writes.
-// cache policy of a buffer access on gfx950: NT (bit 1) streams data that is
+// cache policy of a buffer access on gfx950.  NT (bit 1) streams data that is
 // touched once -- a signal read and a result written -- past the caches, so
 // they stay with data that is reused (the filter, twiddles, LDS spills).
 // Measured on the 1D conv and BFP kernels at every size: +2 to +3.5%, and on
-// a plain copy 5.5 -> 6.2 TB/s.  The four-step middle does not use it: its
-// data is read again by the next launch from the last-level cache.
-enum { POL_DEFAULT = 0, POL_NT = 2 };
+// a plain copy 5.5 -> 6.2 TB/s.
+// WT (SC1, bit 4: device scope) writes a store through the L2 as it is made.
+// The next launch reads the data on any of the 8 XCDs, so a kernel's dirty L2
+// lines are written back at its end in any case; written through, they go out
+// under the kernel, and unlike NT they stay in the last-level cache.  For data
+// the next launch reads, us, default -> WT: four-step 32768 x 50 28.2 -> 18.1, x 301
+// 78.4 -> 74.1, 65536 x 16 22.7 -> 16.3, x 500 247 -> 244, 2^20 x 1 24.9 -> 18.4, x 3 35.9 ->
+// 31.5; conv 2D 256 x 1024 x 8 28.9 -> 25.5, 512 x 512 x 4 19.0 -> 17.3, x 64 137.9 -> 133.0;
+// C2C both ways N = 4096, 2 M points 18.2 -> 14.8, 8 M 46.5 -> 44.2, 17 M 89.1 -> 86.8.
+// For results nothing reads next NT stays: conv N = 1024, 8 M points 24.0, WT 31.4.
+enum { POL_DEFAULT = 0, POL_NT = 2, POL_WT = 16 };
 
 struct Buf {
    __amdgpu_buffer_rsrc_t r;
@@ -319,10 +327,11 @@ struct Buf {
       typedef uint32_t u2 __attribute__((ext_vector_type(2)));
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, soff, POL);
    }
+   template<int POL = POL_DEFAULT>
    __device__ __forceinline__ void st4(float4 v, uint32_t voff, uint32_t soff) const
    {
       typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, POL);
    }
    template<int POL = POL_DEFAULT>
    __device__ __forceinline__ void stu(uint32_t v, uint32_t voff, uint32_t soff) const

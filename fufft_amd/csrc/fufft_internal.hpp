@@ -43,8 +43,9 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 }
 
 // ---- 1D fused pipeline (conv1d.hip) ------------------------------------------------
-// K_APPLY: the split apply, spectra in digit order; K_APPLY_ROWS: the row
-// inverse of the 2D paths, lane-major spectra and no mid operation.
+// K_FWD / K_APPLY: the split forward and apply, spectra in digit order;
+// K_FWD_ROWS / K_APPLY_ROWS: the row forward and inverse of the 2D paths,
+// lane-major spectra and no mid operation.
 // K_CONV_NEAR: K_CONV for signals that the last-level cache keeps: default
 // loads (conv_near).
 // K_FWD_R2 / K_APPLY_R2: the forward half reading two real arrays, the
@@ -71,7 +72,7 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 enum { K_CONV = 0, K_CONV_R2 = 1, K_FWD = 2, K_APPLY = 3, K_FWD_R2 = 4, K_APPLY_R2 = 5,
        K_C2C_FWD = 6, K_C2C_INV = 7, K_PLAN_TAPS = 8, K_CONV_TIMED = 9, K_CONV_MID = 10,
        K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13,
-       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_C2C_FWD_NT = 16, K_C2C_INV_NT = 17 };
+       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_FWD_ROWS = 16 };
 
 // the plans K_CONV_PSF and K_CONV_PSF_DR are built for: radix 16 with whole
 // wavefronts per transform and room for the filter's 32 VGPRs within 128
@@ -112,19 +113,6 @@ constexpr bool conv_near(int64_t n, int64_t batch)
    return conv_near_plan(n) && batch < ((int64_t)128 << 20) / (8 * n);
 }
 
-// A C2C's result is the next call's input (a spectrum on its way back), so it is
-// stored where that call finds it, unless the L2s (32 MiB together) would hold
-// it all, whose lines the end of the kernel then has to write back, or it is
-// more than the 256 MiB last-level cache.  Forward and inverse, us, stores
-// streamed / not: N = 4096, 16 MiB 15.6 / 18.2, 32 MiB 29.6 / 26.5, 48 MiB 42.4 /
-// 36.2, 256 MiB 174.9 / 166.9, 320 MiB 217 / 230, 512 MiB 350 / 365; N = 512, 16 MiB
-// 14.6 / 15.5, 48 MiB 37.3 / 33.9, 256 MiB 171.3 / 164.7, 384 MiB 253 / 259.
-constexpr bool c2c_streams(int64_t n, int64_t batch)
-{
-   const int64_t mib32 = ((int64_t)32 << 20) / (8 * n);      // transforms in 32 MiB
-   return batch < mib32 || batch > 8 * mib32;
-}
-
 // phase timer record of one workgroup (K_CONV_TIMED), TIMER_STRIDE words:
 // [0] HW_ID, [1] XCC_ID, [2] marks, [3] s_memrealtime ticks (100 MHz) from
 // the first mark to the last, [4..5] start (s_memtime, lo / hi),
@@ -145,7 +133,6 @@ struct Conv1dParams {
    uint32_t      scount;   // transform t uses spectrum (t % scount)
    int32_t       mid;      // a registered mid policy id (FUFFT_MID_POLICIES)
    int32_t       fl;       // FLT_DR / FLT_LANE (filter read; K_PLAN_TAPS: layout written)
-   int32_t       sl;       // FLT_DR / FLT_LANE: spectrum K_FWD writes
    float         scale;    // K_PLAN_TAPS: factor applied to the spectrum
    uint32_t*     timing;   // K_CONV_TIMED: TIMER_STRIDE words per workgroup
    uint32_t      timing_groups;   // workgroups that write a record

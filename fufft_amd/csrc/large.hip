@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(256) outer_pass_kernel(const OuterParams p)
    if constexpr(!DIT) twiddle_group<16, CHAIN_SINGLE, 0, 1>(r, w1);
 
 #pragma unroll
-   for(int k = 0; k < 16; k++) io.st2(r[k], voff, k * kst);
+   for(int k = 0; k < 16; k++) io.st2<POL_WT>(r[k], voff, k * kst);
 }
 
 // ---- two outer levels in one pass ----------------------------------------------------
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256) outer2_kernel(const Outer2Params p)
       outer_group<SIGN>(r, tb, j, M2, false);
       const uint32_t vo2 = (j + (uint32_t)k1 * M1) * 8u;
 #pragma unroll
-      for(int q = 0; q < 16; q++) io.st2(r[q], vo2, q * M2 * 8u);
+      for(int q = 0; q < 16; q++) io.st2<POL_WT>(r[q], vo2, q * M2 * 8u);
    } else {
       // level M2 first: group (b = k1, j), taps over k2
       const uint32_t k1 = (uint32_t)hi;
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) outer2_kernel(const Outer2Params p)
       outer_group<SIGN>(r, tb, j + (uint32_t)k2 * M2, M1, true);
       const uint32_t vo2 = (j + (uint32_t)k2 * M2) * 8u;
 #pragma unroll
-      for(int q = 0; q < 16; q++) io.st2(r[q], vo2, q * M1 * 8u);
+      for(int q = 0; q < 16; q++) io.st2<POL_WT>(r[q], vo2, q * M1 * 8u);
    }
 }
 

@@ -20,6 +20,8 @@
 // through 16 KiB of LDS and writes it in output order.  One thread per output
 // point, each reading 8 bytes of a line of its own, had the same lines fetched
 // by several XCDs: N = 4096, 3001 spectra, digit order 112 us; the tiles 34 us, 5.8 TB/s.
+// The filters are written through (POL_WT): the conv reads them next (planning and
+// conv of 8 M points 61.8 -> 59.3 us, 67 M 499 -> 491).
 #include "fufft_device.hpp"
 #include "fufft_internal.hpp"
 
@@ -118,7 +120,7 @@ __global__ void __launch_bounds__(256) plan_tile_kernel(const TileParams p)
 #pragma unroll
    for(int q = 0; q < kPer; q++) {
       const float2 x = lds[tile_slot(threadIdx.x | (q << 8))];
-      ob.st2(make_float2(x.x * p.scale, x.y * p.scale), (so | spread<8, kTileBits - 8>(q << 8, p.tile_out)) * 8u, 0);
+      ob.st2<POL_WT>(make_float2(x.x * p.scale, x.y * p.scale), (so | spread<8, kTileBits - 8>(q << 8, p.tile_out)) * 8u, 0);
    }
 }
 

@@ -43,7 +43,7 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 KINDS = {0: "conv", 1: "conv_r2", 2: "fwd", 3: "apply", 4: "fwd_r2", 5: "apply_r2",
          6: "c2c_fwd", 7: "c2c_inv", 8: "plan_taps", 9: "conv_timed", 10: "conv_mid",
          11: "conv_psf", 12: "conv_psf_dr", 13: "conv_chain", 14: "conv_near", 15: "apply_rows",
-         16: "c2c_fwd_nt", 17: "c2c_inv_nt"}
+         16: "fwd_rows"}
 MIDS = {0: "mul", 1: "conj", 2: "none"}
 LAYOUTS = {0: "xor", 1: "pad", 2: "xchg"}
 FILTERS = {0: "dr", 1: "lane", 2: "bperm"}
@@ -210,12 +210,13 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
     instructions, of one kernel (digit-order filter)."""
     if kind in ("conv_mid", "conv_near"):   # the conv with another cache policy
         kind = "conv"
-    kind = kind.removesuffix("_nt")
     chain = kind == "conv_chain"            # read as the digit-order conv, without its other filter layout
     if chain:
         kind = "conv"
     if kind == "apply_rows":
-        kind, mid = "apply_r2", "none"
+        kind, mid = "apply", "none"
+    if kind == "fwd_rows":
+        kind = "fwd"
     ps = plan(n, v, chain)
     one_dir = sum(pass_ops(v, r, M, n // v) for r, M in ps)
     exchanges = len(ps) - 1

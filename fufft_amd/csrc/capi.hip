@@ -1065,7 +1065,7 @@ int fufft_plan_filter_large_device_f32(const void* in, void* out, int64_t n, int
 // once where the three launches do it three times; the rest run those.  The
 // results are the same bit for bit, so the line is the faster side.  A round of
 // up to 256 transforms (one per CU, where it holds no more) takes some 17 us at
-// n = 16384 and 35 at 32768, full or not, so a last round of a few is left to the
+// n = 16384 and 33 at 32768, full or not, so a last round of a few is left to the
 // three launches.  us a call, shared filter, three buffers in turn, three launches
 // / one / split (whole rounds in one):
 //   n =  8192: 1 11.6 / 9.5, 64 12.4 / 10.1, 200 18.0 / 12.5, 400 32.8 / 18.6;

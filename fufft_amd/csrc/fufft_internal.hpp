@@ -161,7 +161,7 @@ hipError_t launch_conv_wide(const Conv1dParams& p, int n, hipStream_t s);
 // The four-step chain of one outer level in one launch: K_CONV_CHAIN at
 // N = 8192 and 16384, the wide kernel at 32768.  Against the three launches:
 // 8192 x 4000 248.9 -> 124.8 us, 16384 x 300 43.4 -> 36.2, 32768 x 256 68.5 ->
-// 52.5; the batches that take it are chain_batch's choice (capi.hip).
+// 47.4; the batches that take it are chain_batch's choice (capi.hip).
 constexpr bool conv_chain_plan(int64_t n, int v) { return v == 16 && (n == 8192 || n == 16384 || n == CONV_WIDE_N); }
 hipError_t launch_conv_wide_chain(const Conv1dParams& p, int n, hipStream_t s);
 

@@ -150,7 +150,7 @@ def decode_name(name: str) -> dict | None:
         # big: blocks of more than 64 points (LDS rendezvous of the block maxima)
         return {"family": "bfp", "n": n, "v": v, "layout": LAYOUTS[lay],
                 "kind": "conv_blocks" if big else "conv", "mid": MIDS[mid]}
-    # the N = 16384 / 32768 conv (wide.hip): 32 values per lane, float exchanges;
+    # the N = 16384 / 32768 conv (wide.hip): 32 values per lane, exchanges in two halves;
     # "wide_chain": the four-step chain's pass order
     m = re.search(r"conv_wide_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb([01])E", name)
     if m:
@@ -265,8 +265,8 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
 def model_wide(mid: str = "mul", filt: str = "lane", n: int = 32768, v: int = 32, chain: bool = False) -> dict:
     """The N = 16384 / 32768 conv (wide.hip): the radix-16 plan with V/R groups
     per lane in every pass (8 / 4 in the radix-4 / radix-8 lead, 2 in the
-    radix-16 passes), no kept chain; each exchange writes and reads both float
-    components of the lane's V values (V 8-byte equivalents each way); the
+    radix-16 passes), no kept chain, one twiddle chain for both halves of a
+    later pass (the compiler finds them equal); each exchange writes and reads the lane's V values once; the
     filter as V/2 16-byte loads (V 8-byte ones in bperm).  A lead pass of more
     than 4 groups per lane reads its base twiddles again for the inverse."""
     ps = plan(n, 16, chain)
@@ -324,7 +324,7 @@ def conv_rows(rows=None) -> list:
         n, v = d["n"], d["v"]
         t = n // v
         threads = t if t >= 128 else 256
-        # the wide kernel's float buffer: N + N/16 slots of 4 bytes
+        # the wide kernel's buffer: N/2 + N/32 slots of 8 bytes
         wide = d["family"] in ("wide", "wide_chain")
         lds = (n + n // 16) * 4 if wide else lds_bytes_conv(n, v, d["layout"])
         occ = occupancy(r["meta"]["vgpr_count"], r["meta"].get("agpr_count", 0), lds, threads // 64)

@@ -4,7 +4,7 @@ The compute path is the in-tree HIP library ``libfufft_amd.so`` (built by
 ``fufft_amd.build``).  There is no fallback: if the library is missing, import
 fails loudly.  Device buffers are torch tensors on ``cuda`` (ROCm); every
 launch wrapper checks their dtype, contiguity, size and device before the
-call (``_dev``), and launches on torch's current stream unless given one.
+call (``_ptrs``), and launches on torch's current stream unless given one.
 
 torch is imported before the library is loaded so that both share torch's HIP
 runtime (torch bundles its own ``libamdhip64.so.7``; the loader then resolves
@@ -149,8 +149,11 @@ if torch is not None:
     # the reads every launch makes, without torch.cuda's Python layer (which
     # initialises the GPU on first use: a tensor that is on one has done that)
     _TENSOR = torch.Tensor
-    _current_device = torch._C._cuda_getDevice
-    _current_raw_stream = torch._C._cuda_getCurrentRawStream
+    # a torch build without GPU support lacks these two bindings; the host
+    # planners work there, and a launch is refused by the public calls
+    _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+    _current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                                  lambda device: torch.cuda.current_stream(device).cuda_stream)
 
 
 def _check_shape(x, name: str, nbytes: int, kind: str) -> None:
@@ -305,7 +308,7 @@ def get_twiddles(device: int = 0) -> str:
 
 
 # ---- launches ------------------------------------------------------------------------
-# Each wrapper checks its tensors (_dev) against the sizes the call implies
+# Each wrapper checks its tensors (_ptrs) against the sizes the call implies
 # before the library sees them; the library then checks sizes, strides,
 # enums and alignment again and returns a status, raised as FufftError.
 

@@ -8,6 +8,9 @@ Python, before any GPU call.  Also checked: every variant default is "auto",
 so a filter planned with the defaults matches a launch with the defaults.
 """
 import inspect
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -156,3 +159,27 @@ def test_host_bfp_codecs_check_their_arrays(ff):
         ff.bfp_scaled_dequantize(q, np.ones(1, dtype=np.float32), n)
     with pytest.raises(ValueError, match="whole transforms"):
         ff.bfp_scaled_dequantize(q[:-2], np.ones(2, dtype=np.float32), n)
+
+
+def test_import_on_a_torch_build_without_gpu_support():
+    """Such a build of torch lacks the bindings that the launches read the
+    device and stream with; the package imports all the same, its host
+    planners run, and a launch still refuses a host tensor."""
+    code = """
+import torch
+for name in ("_cuda_getDevice", "_cuda_getCurrentRawStream"):
+    delattr(torch._C, name)
+import numpy as np
+import fufft_amd as ff
+assert ff.plan_filter(np.ones(256, np.complex64), 256).shape == (256,)
+x = torch.zeros(256, dtype=torch.complex64)
+try:
+    ff.conv(x, x, torch.zeros_like(x), n=256, batch=1)
+except ValueError as e:
+    assert "not in GPU memory" in str(e)
+else:
+    raise AssertionError("a host tensor was not refused")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=Path(__file__).resolve().parent.parent,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr

@@ -337,16 +337,30 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    }
 }
 
+// The workgroup runs conv_iters groups of transforms where the kernel loops, one
+// in any other, and that one trip is a loop too: the compiler then issues the
+// argument loads together, ahead of the first wait; in straight code, or with a
+// function between the two, some of them come after it, or deep in the body
+// (radix 8).  us, straight / loop, 2^27 points: conv N = 4096 lane-major 391 / 388;
+// digit order at radix 16, N = 1024 391 / 388, 4096 407 / 402, 8192 500 / 492; split
+// forward N = 4096 442 / 425 (33 M points 122 / 113).  Two kinds are faster
+// straight: the split apply (a spectrum and a filter per transform, N = 1024 570
+// / 604; one spectrum, N = 4096 373 / 387) and the near conv (N = 1024, 8 M points
+// 23.65 / 23.95).
+template<int KIND>
+constexpr bool conv_straight() { return KIND == K_APPLY || KIND == K_CONV_NEAR; }
+
 template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_loops<N, KIND>()) {
-#pragma unroll 1
-      for(uint32_t it = 0; it < p.iters; it++)
-         conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x * p.iters + it);
-   } else {
+   if constexpr(conv_straight<KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x);
+   } else {
+      const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
+#pragma unroll 1
+      for(uint32_t it = 0; it < iters; it++)
+         conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x * iters + it);
    }
 }
 
@@ -355,12 +369,13 @@ template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_bperm_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_loops<N, KIND>()) {
-#pragma unroll 1
-      for(uint32_t it = 0; it < p.iters; it++)
-         conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x * p.iters + it);
-   } else {
+   if constexpr(conv_straight<KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x);
+   } else {
+      const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
+#pragma unroll 1
+      for(uint32_t it = 0; it < iters; it++)
+         conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x * iters + it);
    }
 }
 

@@ -1,4 +1,4 @@
-"""The cache policy of the conv's loads (signals under 128 MiB or not) and of the
+"""The cache policy of the conv's loads (signals of up to 64 MiB or more) and of the
 C2C's stores (results of 32 to 256 MiB or not) is the launch's choice by size, each
 with a kernel of its own.  On both sides of the line, and beside it, a batch
 gives what its parts give in small calls (parity of those with the oracle:
@@ -29,7 +29,7 @@ def _signals(dev, n, batch):
 def test_conv_loads(dev, n, variant, layout, past):
     import torch
     import fufft_amd as ff
-    batch = (128 << 20) // (8 * n) + past
+    batch = (64 << 20) // (8 * n) + past
     print(f"case conv policy n={n} {variant} {layout} batch={batch}", flush=True)
     x, gen = _signals(dev, n, batch)
     f = torch.randn(n, dtype=torch.complex64, device=dev, generator=gen)

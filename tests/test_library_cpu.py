@@ -431,3 +431,29 @@ def test_cpp_plan_objects_build_and_reject_bad_arguments(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, (out.returncode, out.stdout, out.stderr)
     assert out.stdout.startswith("ok")
+
+
+def test_near_conv_leaves_room_for_the_next_batches(tmp_path):
+    """The rule that gives a conv default loads (conv_near) holds only where
+    four batches of its signals fit the 256 MiB last-level cache together: a
+    program that convolves them in turn otherwise has each one pushed out
+    before it comes back.  No batch size of N >= 16384 takes it."""
+    import shutil
+    import subprocess
+    rocm = Path("/opt/rocm")
+    if shutil.which("g++") is None or not (rocm / "include" / "hip" / "hip_runtime.h").exists():
+        pytest.skip("g++ or the HIP headers are not available")
+    src = tmp_path / "near.cpp"
+    src.write_text('''
+#include "fufft_internal.hpp"
+constexpr int64_t most(int64_t n) { int64_t b = 0; while(fufft::conv_near(n, b + 1)) b++; return b; }
+constexpr bool fits(int64_t n) { return most(n) > 0 && 4 * most(n) * n * 8 <= (int64_t)256 << 20; }
+static_assert(fits(2048) && fits(4096) && fits(8192), "four batches in the cache");
+static_assert(!fufft::conv_near(256, (65 << 20) / (8 * 256)) && !fufft::conv_near(512, (96 << 20) / (8 * 512)), "");
+static_assert(most(16384) == 0 && most(32768) == 0, "one policy");
+int main() { return 0; }
+''')
+    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-loop-limit=10000000", "-D__HIP_PLATFORM_AMD__",
+                        f"-I{ROOT / 'include'}", f"-I{ROOT / 'fufft_amd' / 'csrc'}", f"-I{rocm / 'include'}", str(src)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr

@@ -113,15 +113,19 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // N = 16384, where writing through measured 2-10% faster (8 M points 52.0 -> 46.4
    // us).  The loads stream too where the signals are more than the last-level
    // cache keeps.  The split forward keeps the default: its digit-order stores
-   // are 16-byte pieces that the L2 puts together.
+   // are 16-byte pieces that the L2 puts together.  So does the real conv at N =
+   // 256, whose 16 lanes store 64 bytes, half a line (us, default / streamed, real
+   // pairs in turn: one of 16 M points 43.9 / 49.0, three 53.2 / 56.2; 134 M 386 / 403).
+   constexpr int  EL_IN  = REAL_IN ? 4 : 8;
+   constexpr int  EL_OUT = REAL_OUT ? 4 : 8;
+   constexpr bool LINES = (T < 64 ? T : 64) * EL_OUT >= 128;   // a wavefront's store covers whole lines
    constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
    constexpr bool KEPT = KIND == K_CONV_MID || KIND == K_FWD_ROWS || KIND == K_FWD_R2 || KIND == K_APPLY_ROWS ||
                          KIND == K_APPLY_R2 || C2C_FWD || C2C_INV || (KIND == K_CONV && N == 16384);
    constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
    constexpr int  ST_POL = KEPT ? POL_WT
-                         : (ONCE || KIND == K_CONV_NEAR || KIND == K_CONV_R2 || KIND == K_APPLY) ? POL_NT : POL_DEFAULT;
-   constexpr int  EL_IN     = REAL_IN ? 4 : 8;
-   constexpr int  EL_OUT    = REAL_OUT ? 4 : 8;
+                         : (ONCE || KIND == K_CONV_NEAR || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY) ? POL_NT
+                                                                                                            : POL_DEFAULT;
 
    extern __shared__ float2 lds[];
    const int slot = threadIdx.x / T;

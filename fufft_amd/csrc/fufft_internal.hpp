@@ -110,8 +110,8 @@ constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 // both together, 64 MiB 185 / 192, 120 MiB 204 / 220; with 128 MiB 49.5 / 44.8.
 // The other single-launch kinds have one policy.  Stores streamed, loads not:
 // the split apply (N = 512 / 4096 / 8192, 8 M points 29.3 / 33.6 / 38.9 -> 24.3 / 26.9
-// / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv (8 M, N = 256 / 4096 30.9 /
-// 31.9 -> 26.0 / 26.5) and the small images; both streamed: one filter per signal,
+// / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv from N = 512 (8 M, N = 4096 31.9
+// -> 26.5) and the small images; both streamed: one filter per signal,
 // the four-step chain and N >= 16384, which measured best or even so.
 constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
 constexpr bool conv_near(int64_t n, int64_t batch)

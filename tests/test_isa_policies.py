@@ -1,0 +1,50 @@
+"""Cache policies of the compiled kernels' loads and stores, read from this
+build's own gfx950 code: a buffer access streams past the caches (nt), is
+written through the L2 (sc1) or has the default policy (neither)."""
+import re
+import subprocess
+
+import pytest
+
+from fufft_amd import isa_report as R
+
+pytestmark = pytest.mark.skipif(not R.tools_available() or not list(R.OBJ.glob("*.o")),
+                                reason="needs this build's objects and the ROCm LLVM tools")
+
+
+def policies(obj, workdir):
+    """kernel name -> list of (opcode, policy) of its buffer accesses, in order"""
+    text = subprocess.run([str(R.LLVM / "llvm-objdump"), "-d", "--no-show-raw-insn", str(R.code_object(obj, workdir))],
+                          check=True, capture_output=True, text=True).stdout
+    out, name = {}, None
+    for line in text.splitlines():
+        m = re.match(r"^[0-9a-f]+ <(\S+)>:", line)
+        if m:
+            name = m.group(1)
+            out[name] = []
+            continue
+        m = re.search(r"\b(buffer_(?:load|store)_\w+) ([^/]*)", line)
+        if m and name:
+            mods = set(m.group(2).split()) & {"nt", "sc1"}
+            out[name].append((m.group(1), "+".join(sorted(mods)) or "default"))
+    return out
+
+
+@pytest.fixture(scope="module")
+def conv1d(tmp_path_factory):
+    return policies(R.OBJ / "conv1d.o", tmp_path_factory.mktemp("co1"))
+
+
+def kernel(n, v, kind, mid=0, layout=2):
+    return f"_ZN5fufft13conv1d_kernelILi{n}ELi{v}ELi{layout}ELi{kind}ELi{mid}EEEvNS_12Conv1dParamsE"
+
+
+def stores(accesses, width="dword"):
+    return {p for op, p in accesses if op.startswith("buffer_store_" + width)}
+
+
+@pytest.mark.parametrize("n,v,policy", [(256, 16, "default"), (512, 16, "nt"), (512, 8, "nt"), (4096, 16, "nt")])
+def test_real_conv_streams_whole_lines_only(conv1d, n, v, policy):
+    """At N = 256 sixteen lanes store 64 bytes of a real result at a time: half a
+    line, which a streamed store sends out by itself."""
+    assert stores(conv1d[kernel(n, v, 1)]) == {policy}

@@ -698,7 +698,8 @@ int fufft_c2c_f32(const void* in, void* out, int64_t n, int64_t batch, int direc
    if((st = current_table(&p.tw)) != FUFFT_OK) return st;
    p.in0 = in; p.out0 = out; p.ntrans = (uint32_t)batch;
    p.fcount = 1; p.scount = 1; p.mid = FUFFT_MID_NONE; p.fl = FUFFT_LAYOUT_DR;
-   return run_conv1d(direction == FUFFT_FORWARD ? K_C2C_FWD : K_C2C_INV, (int)n, v, p, stream);
+   const int kind = direction == FUFFT_INVERSE ? K_C2C_INV : c2c_far(n, batch) ? K_C2C_FAR : K_C2C_FWD;
+   return run_conv1d(kind, (int)n, v, p, stream);
 }
 
 // ---- filter planning on the device -------------------------------------------------------

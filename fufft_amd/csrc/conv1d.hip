@@ -93,7 +93,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    constexpr bool FROM_ROWS = KIND == K_APPLY_ROWS || KIND == K_APPLY_R2;   // 2D rows: lane-major spectra
    constexpr bool FROM_SPEC = KIND == K_APPLY || FROM_ROWS;
    constexpr bool TO_SPEC   = KIND == K_FWD || KIND == K_FWD_ROWS || KIND == K_FWD_R2;
-   constexpr bool C2C_FWD   = KIND == K_C2C_FWD;
+   constexpr bool C2C_FWD   = KIND == K_C2C_FWD || KIND == K_C2C_FAR;
    constexpr bool C2C_INV   = KIND == K_C2C_INV;
    constexpr bool PLAN      = KIND == K_PLAN_TAPS;
    constexpr bool TIMED     = KIND == K_CONV_TIMED;
@@ -121,11 +121,11 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    constexpr bool LINES = (T < 64 ? T : 64) * EL_OUT >= 128;   // a wavefront's store covers whole lines
    constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
    constexpr bool KEPT = KIND == K_CONV_MID || KIND == K_FWD_ROWS || KIND == K_FWD_R2 || KIND == K_APPLY_ROWS ||
-                         KIND == K_APPLY_R2 || C2C_FWD || C2C_INV || (KIND == K_CONV && N == 16384);
+                         KIND == K_APPLY_R2 || KIND == K_C2C_FWD || C2C_INV || (KIND == K_CONV && N == 16384);
    constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
    constexpr int  ST_POL = KEPT ? POL_WT
-                         : (ONCE || KIND == K_CONV_NEAR || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY) ? POL_NT
-                                                                                                            : POL_DEFAULT;
+                         : (ONCE || KIND == K_C2C_FAR || KIND == K_CONV_NEAR || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY)
+                              ? POL_NT : POL_DEFAULT;
 
    extern __shared__ float2 lds[];
    const int slot = threadIdx.x / T;
@@ -470,6 +470,9 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
          return p.mid == MID_NONE ? launch_one<N, V, LAYOUT, K_APPLY_R2, MID_NONE>(p, s)
                                   : hipErrorInvalidValue;
       case K_C2C_FWD:   return launch_one<N, V, LAYOUT, K_C2C_FWD, MID_NONE>(p, s);
+      case K_C2C_FAR:
+         if constexpr(c2c_far_plan(N)) return launch_one<N, V, LAYOUT, K_C2C_FAR, MID_NONE>(p, s);
+         else                          return hipErrorInvalidValue;
       case K_C2C_INV:   return launch_one<N, V, LAYOUT, K_C2C_INV, MID_NONE>(p, s);
       case K_PLAN_TAPS: return launch_one<N, V, LAYOUT, K_PLAN_TAPS, MID_NONE>(p, s);
       case K_CONV_TIMED:

@@ -47,7 +47,7 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 // K_FWD_ROWS / K_APPLY_ROWS: the row forward and inverse of the 2D paths,
 // lane-major spectra and no mid operation.
 // K_CONV_NEAR: K_CONV for signals that the last-level cache keeps: default
-// loads (conv_near).
+// loads (conv_near).  K_C2C_FAR: K_C2C_FWD with streamed stores (c2c_far).
 // K_FWD_R2 / K_APPLY_R2: the forward half reading two real arrays, the
 // inverse half writing two real arrays (2D two-for-one rows).
 // K_C2C_FWD / K_C2C_INV: natural order in and out (forward DIF + digit ->
@@ -72,7 +72,7 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 enum { K_CONV = 0, K_CONV_R2 = 1, K_FWD = 2, K_APPLY = 3, K_FWD_R2 = 4, K_APPLY_R2 = 5,
        K_C2C_FWD = 6, K_C2C_INV = 7, K_PLAN_TAPS = 8, K_CONV_TIMED = 9, K_CONV_MID = 10,
        K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13,
-       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_FWD_ROWS = 16 };
+       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_FWD_ROWS = 16, K_C2C_FAR = 17 };
 
 // the plans K_CONV_PSF and K_CONV_PSF_DR are built for: radix 16 with whole
 // wavefronts per transform and room for the filter's 32 VGPRs within 128
@@ -117,6 +117,17 @@ constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
 constexpr bool conv_near(int64_t n, int64_t batch)
 {
    return conv_near_plan(n) && batch <= ((int64_t)64 << 20) / (8 * n);
+}
+
+// K_C2C_FAR: spectra of more than 512 MiB at N = 256.  Nothing of them is in the
+// caches when the next launch reads it, and at this size alone streaming is then
+// the faster.  us, written through / streamed: 67 M points 173 / 173, 84 M 221.5 /
+// 218, 101 M 270 / 264, 134 M 369 / 357; N = 1024, 134 M 344 / 349; N = 4096 and the
+// inverses even or faster written through.
+constexpr bool c2c_far_plan(int64_t n) { return n == 256; }
+constexpr bool c2c_far(int64_t n, int64_t batch)
+{
+   return c2c_far_plan(n) && batch > ((int64_t)512 << 20) / (8 * n);
 }
 
 // phase timer record of one workgroup (K_CONV_TIMED), TIMER_STRIDE words:

@@ -48,3 +48,13 @@ def test_real_conv_streams_whole_lines_only(conv1d, n, v, policy):
     """At N = 256 sixteen lanes store 64 bytes of a real result at a time: half a
     line, which a streamed store sends out by itself."""
     assert stores(conv1d[kernel(n, v, 1)]) == {policy}
+
+
+@pytest.mark.parametrize("n,v", [(256, 16), (512, 8), (1024, 16), (4096, 8), (4096, 16), (16384, 16)])
+def test_c2c_spectra_are_written_through(conv1d, n, v):
+    """What the inverse reads back is written through; at N = 256 the forward has
+    a kernel that streams, for spectra of more than 512 MiB."""
+    assert stores(conv1d[kernel(n, v, 6, mid=2)]) == {"sc1"}
+    assert stores(conv1d[kernel(n, v, 7, mid=2)]) == {"sc1"}
+    far = kernel(n, v, 17, mid=2)
+    assert (stores(conv1d[far]) == {"nt"}) if n == 256 else (far not in conv1d)

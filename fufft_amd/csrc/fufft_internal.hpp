@@ -92,7 +92,7 @@ constexpr bool conv_psf_dr_plan(int n, int v) { return v == 16 && (n == 2048 || 
 // 213.3, so those sizes keep the plain kernel.
 constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 
-// K_CONV_NEAR runs the conv whose signals take at most a quarter of the 256 MiB
+// K_CONV_NEAR runs the conv whose signals take up to 80 MiB of the 256 MiB
 // last-level cache.  What a program convolves was mostly just written, or is
 // convolved again, and a default load keeps it there, where a streaming one
 // has the next pass fetch it from HBM.  Three states in turn, us, loads and
@@ -101,11 +101,11 @@ constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 //     29.3 / 23.8 / 29.9;
 //   N = 512: 8 M 26.0 / 21.7 / 27.7; N = 4096: 8 M 29.8 / 26.1 / 30.0; N = 8192: 8 M
 //     38.1 / 36.2 / 40.6; N = 16384 and 32768 even.
-// The line lies where four such batches still fit.  Loads streamed / not, N = 1024,
-// one to four batches in turn: 64 MiB 26.2 / 24.2, 27.4 / 24.4, 28.0 / 24.6, 27.6 /
-// 25.9; 80 MiB 32.5 / 29.2, 33.5 / 29.5, 33.5 / 30.1, 33.5 / 35.7; 96 MiB 38.9 /
-// 34.2, 39.8 / 34.7, 40.3 / 40.7, 39.1 / 41.5 (N = 512: 39.3 / 42.3 for three).  Sixteen
-// of 64 MiB in turn 29.0 / 29.4.  Signals that come from HBM to a cache full of
+// The line lies where three such batches still fit.  Loads streamed / not, N =
+// 1024, one to four batches in turn: 64 MiB 26.2 / 24.2, 27.4 / 24.4, 28.0 / 24.6,
+// 27.6 / 25.9; 80 MiB 32.5 / 29.2, 33.5 / 29.5, 33.5 / 30.1, 33.5 / 35.7; 96 MiB 38.9
+// / 34.2, 39.8 / 34.7, 40.3 / 40.7, 39.1 / 41.5 (N = 512: 39.3 / 42.3 for three).
+// Sixteen of 64 MiB in turn 29.0 / 29.4.  Signals that come from HBM to a cache full of
 // results push those out under the conv: with 1 GiB written before each call,
 // both together, 64 MiB 185 / 192, 120 MiB 204 / 220; with 128 MiB 49.5 / 44.8.
 // The other single-launch kinds have one policy.  Stores streamed, loads not:
@@ -116,7 +116,7 @@ constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
 constexpr bool conv_near(int64_t n, int64_t batch)
 {
-   return conv_near_plan(n) && batch <= ((int64_t)64 << 20) / (8 * n);
+   return conv_near_plan(n) && batch <= ((int64_t)80 << 20) / (8 * n);
 }
 
 // K_C2C_FAR: spectra of more than 512 MiB at N = 256.  Nothing of them is in the

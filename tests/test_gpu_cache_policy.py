@@ -1,4 +1,4 @@
-"""The cache policy of the conv's loads (signals of up to 64 MiB, with a kernel of
+"""The cache policy of the conv's loads (signals of up to 80 MiB, with a kernel of
 its own, or more) and of the C2C forward's stores at N = 256 (spectra of up to
 512 MiB or more) is chosen by size.  On both sides of the line, and beside it,
 a batch gives what its parts give in small calls (parity of those with the
@@ -30,7 +30,7 @@ def _signals(dev, n, batch):
 def test_conv_loads(dev, n, variant, layout, past):
     import torch
     import fufft_amd as ff
-    batch = (64 << 20) // (8 * n) + past
+    batch = (80 << 20) // (8 * n) + past
     print(f"case conv policy n={n} {variant} {layout} batch={batch}", flush=True)
     x, gen = _signals(dev, n, batch)
     f = torch.randn(n, dtype=torch.complex64, device=dev, generator=gen)

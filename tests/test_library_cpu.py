@@ -435,7 +435,7 @@ def test_cpp_plan_objects_build_and_reject_bad_arguments(tmp_path):
 
 def test_near_conv_leaves_room_for_the_next_batches(tmp_path):
     """The rule that gives a conv default loads (conv_near) holds only where
-    four batches of its signals fit the 256 MiB last-level cache together: a
+    three batches of its signals fit the 256 MiB last-level cache together: a
     program that convolves them in turn otherwise has each one pushed out
     before it comes back.  No batch size of N >= 16384 takes it."""
     import shutil
@@ -447,9 +447,9 @@ def test_near_conv_leaves_room_for_the_next_batches(tmp_path):
     src.write_text('''
 #include "fufft_internal.hpp"
 constexpr int64_t most(int64_t n) { int64_t b = 0; while(fufft::conv_near(n, b + 1)) b++; return b; }
-constexpr bool fits(int64_t n) { return most(n) > 0 && 4 * most(n) * n * 8 <= (int64_t)256 << 20; }
-static_assert(fits(2048) && fits(4096) && fits(8192), "four batches in the cache");
-static_assert(!fufft::conv_near(256, (65 << 20) / (8 * 256)) && !fufft::conv_near(512, (96 << 20) / (8 * 512)), "");
+constexpr bool fits(int64_t n) { return most(n) > 0 && 3 * most(n) * n * 8 <= (int64_t)256 << 20; }
+static_assert(fits(2048) && fits(4096) && fits(8192), "three batches in the cache");
+static_assert(!fufft::conv_near(256, (88 << 20) / (8 * 256)) && !fufft::conv_near(512, (96 << 20) / (8 * 512)), "");
 static_assert(most(16384) == 0 && most(32768) == 0, "one policy");
 int main() { return 0; }
 ''')

@@ -399,9 +399,15 @@ small2d_kernel(const Small2dParams p)
 #pragma unroll
       for(int q = 0; q < 8; q++) wb.st2<POL_NT>(lds[stage_slot(q * 64 + wl)], wl * 8u, q * 512);
    } else {
+      // rows of 64 points are stored 64 bytes, half a line, at a time; streamed
+      // halves go out by themselves, which images of up to 16 rows do not hide.  us,
+      // default / streamed: 8 x 64, one batch of 16 M points 42.8 / 49.1, three in turn
+      // 54.3 / 59.6, 134 M 417 / 433; 16 x 64 three of 16 M 60.2 / 64.9, 134 M 466 / 476;
+      // 32 x 64 three of 16 M 65.6 / 65.1, 33 M 124.3 / 105.0
+      constexpr int ST_POL = W == 64 && H <= 16 ? POL_DEFAULT : POL_NT;
       const Buf ob(static_cast<char*>(p.out) + (size_t)t * BYTES, live ? BYTES : 0u);
 #pragma unroll
-      for(int q = 0; q < 8; q++) ob.st2<POL_NT>(r[q], (uint32_t)(rr * W + rl) * 8u, q * TW * 8);
+      for(int q = 0; q < 8; q++) ob.st2<ST_POL>(r[q], (uint32_t)(rr * W + rl) * 8u, q * TW * 8);
    }
 }
 

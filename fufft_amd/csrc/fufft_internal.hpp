@@ -105,14 +105,15 @@ constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 // 1024, one to four batches in turn: 64 MiB 26.2 / 24.2, 27.4 / 24.4, 28.0 / 24.6,
 // 27.6 / 25.9; 80 MiB 32.5 / 29.2, 33.5 / 29.5, 33.5 / 30.1, 33.5 / 35.7; 96 MiB 38.9
 // / 34.2, 39.8 / 34.7, 40.3 / 40.7, 39.1 / 41.5 (N = 512: 39.3 / 42.3 for three).
-// Sixteen of 64 MiB in turn 29.0 / 29.4.  Signals that come from HBM to a cache full of
-// results push those out under the conv: with 1 GiB written before each call,
-// both together, 64 MiB 185 / 192, 120 MiB 204 / 220; with 128 MiB 49.5 / 44.8.
+// Sixteen of 64 MiB in turn 29.0 / 29.4.  Signals that come from HBM to a cache
+// full of results push those out under the conv: with 1 GiB written before each
+// call, both together, 64 MiB 185 / 192, 120 MiB 204 / 220; with 128 MiB 49.5 / 44.8.
 // The other single-launch kinds have one policy.  Stores streamed, loads not:
 // the split apply (N = 512 / 4096 / 8192, 8 M points 29.3 / 33.6 / 38.9 -> 24.3 / 26.9
-// / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv from N = 512 (8 M, N = 4096 31.9
-// -> 26.5) and the small images; both streamed: one filter per signal,
-// the four-step chain and N >= 16384, which measured best or even so.
+// / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv from N = 512 on (8 M,
+// N = 4096 31.9 -> 26.5) and the small images but 8 x 64 and 16 x 64; both streamed:
+// one filter per signal, the four-step chain and N >= 16384, which measured best
+// or even so.
 constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
 constexpr bool conv_near(int64_t n, int64_t batch)
 {

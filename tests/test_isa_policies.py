@@ -58,3 +58,14 @@ def test_c2c_spectra_are_written_through(conv1d, n, v):
     assert stores(conv1d[kernel(n, v, 7, mid=2)]) == {"sc1"}
     far = kernel(n, v, 17, mid=2)
     assert (stores(conv1d[far]) == {"nt"}) if n == 256 else (far not in conv1d)
+
+
+@pytest.mark.parametrize("h,w,policy", [(8, 64, "default"), (16, 64, "default"), (32, 64, "nt"), (64, 64, "nt"),
+                                        (8, 32, "nt"), (8, 128, "nt"), (512, 16, "nt")])
+def test_small_images_of_half_line_stores(tmp_path, h, w, policy):
+    """Rows of 64 points are stored half a line at a time; images of few such rows
+    leave the halves to the L2 to put together."""
+    got = policies(R.OBJ / "conv2d.o", tmp_path)
+    for mid in (0, 1, 2):
+        name = f"_ZN5fufft14small2d_kernelILi{h}ELi{w}ELi{mid}EEEvNS_13Small2dParamsE"
+        assert stores(got[name]) == {policy}

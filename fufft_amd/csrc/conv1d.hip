@@ -121,7 +121,8 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    constexpr bool LINES = (T < 64 ? T : 64) * EL_OUT >= 128;   // a wavefront's store covers whole lines
    constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
    constexpr bool KEPT = KIND == K_CONV_MID || KIND == K_FWD_ROWS || KIND == K_FWD_R2 || KIND == K_APPLY_ROWS ||
-                         KIND == K_APPLY_R2 || KIND == K_C2C_FWD || C2C_INV || (KIND == K_CONV && N == 16384);
+                         KIND == K_APPLY_R2 || KIND == K_C2C_FWD || C2C_INV ||
+                         ((KIND == K_CONV || TIMED) && N == 16384);
    constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
    constexpr int  ST_POL = KEPT ? POL_WT
                          : (ONCE || KIND == K_C2C_FAR || KIND == K_CONV_NEAR || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY)
@@ -214,8 +215,16 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
             r[q] = make_float2(xb.ld1<LD_POL>(lane_pos * 4u, q * T * 4), yb.ld1<LD_POL>(lane_pos * 4u, q * T * 4));
       } else {
          const Buf xb(static_cast<const char*>(p.in0) + wb, WB);
+         // the timer reads as the conv of this batch does, K_CONV_NEAR or K_CONV
+         bool near = false;
+         if constexpr(TIMED) near = conv_near(N, p.ntrans);
+         if(TIMED && near) {
 #pragma unroll
-         for(int q = 0; q < V; q++) r[q] = xb.ld2<LD_POL>(lane_pos * 8u, q * T * 8);
+            for(int q = 0; q < V; q++) r[q] = xb.ld2(lane_pos * 8u, q * T * 8);
+         } else {
+#pragma unroll
+            for(int q = 0; q < V; q++) r[q] = xb.ld2<LD_POL>(lane_pos * 8u, q * T * 8);
+         }
       }
       if constexpr(PSF) {
          // each signal's own filter is a third stream from HBM: issued here,

@@ -259,6 +259,8 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
     # digit-order and pair spectrum stores take one code path (the offsets are selected); a
     # bperm filter read has kernels of its own (conv1d_bperm_kernel, bfp_bperm_kernel).
     untaken_loads = v // 2 if (kind in ("conv", "conv_r2", "conv_timed", "apply", "apply_r2") and mid != "none") else 0
+    if kind == "conv_timed" and n <= 8192:
+        untaken_loads += v               # the signal read with the other cache policy (conv_near)
     untaken = {"loads": untaken_loads, "stores": v if kind == "plan_taps" else 0}
     return {"fp32_arith_per_lane": arith, "lds_access_8B_per_lane": lds, "vmem_loads_per_wave": loads,
             "vmem_stores_per_wave": stores, "untaken_branch": untaken, "passes": ps}

@@ -199,7 +199,13 @@ int fufft_conv_f32(const void* in, const void* filt, int64_t filt_stride,
  * the workgroup's outstanding memory operations and a workgroup barrier, then
  * reads the shader clock (s_memtime), so the timed launch is slower than the
  * untimed one; read proportions and confirm totals against fufft_conv_f32.
- * The output is bit-identical to fufft_conv_f32.
+ * The output is bit-identical to fufft_conv_f32, and signal and result are read
+ * and written with the cache policies that fufft_conv_f32 takes for a shared
+ * filter of that batch in the plan's own kernel.  Always one group of transforms
+ * per workgroup (fufft_conv_f32 runs several in turn at n = 16384), the filter
+ * read at the mid operation (one filter per signal: fufft_conv_f32 issues those
+ * loads earlier at some sizes), and not the 32-values-per-lane kernel that
+ * fufft_conv_f32 takes at n = 16384 for a shared lane-major filter.
  * Workgroup g (transforms [g*tpw, (g+1)*tpw), tpw from
  * fufft_transforms_per_workgroup) writes, for g < timing_groups, the
  * FUFFT_TIMER_STRIDE words at timing + g*FUFFT_TIMER_STRIDE (device memory):

@@ -60,6 +60,22 @@ def test_c2c_spectra_are_written_through(conv1d, n, v):
     assert (stores(conv1d[far]) == {"nt"}) if n == 256 else (far not in conv1d)
 
 
+@pytest.mark.parametrize("n,v", [(256, 16), (512, 8), (1024, 16), (4096, 16), (4096, 8), (8192, 8), (16384, 16)])
+def test_phase_timer_has_the_policies_of_the_conv(conv1d, n, v):
+    """The timed kernel stores as the conv of the same plan does, and where that
+    has a kernel with default loads for small batches, it holds both reads."""
+    layout = 1 if (n, v) == (8192, 8) else 2
+    conv, timed = (conv1d[kernel(n, v, k, layout=layout)] for k in (0, 9))
+    assert stores(timed, "dwordx2") == stores(conv, "dwordx2") == ({"sc1"} if n == 16384 else {"nt"})
+    near = kernel(n, v, 14, layout=layout)
+    assert (near in conv1d) == (n <= 8192)
+    streamed = sum(p == "nt" for op, p in timed if op == "buffer_load_dwordx2")
+    default = sum(p == "default" for op, p in timed if op == "buffer_load_dwordx2")
+    plain = sum(p == "default" for op, p in conv if op == "buffer_load_dwordx2")
+    assert streamed == v
+    assert default == plain + (v if n <= 8192 else 0)
+
+
 @pytest.mark.parametrize("h,w,policy", [(8, 64, "default"), (16, 64, "default"), (32, 64, "nt"), (64, 64, "nt"),
                                         (8, 32, "nt"), (8, 128, "nt"), (512, 16, "nt")])
 def test_small_images_of_half_line_stores(tmp_path, h, w, policy):

@@ -62,12 +62,12 @@ namespace {
 template<int N, bool CHAIN = false>
 using WPlan = Plan<N, 32, 16, CHAIN>;
 
-// Slot layouts of one half's positions, 8-byte slots.  gfx950 serves the 8-byte LDS
-// forms 32 lanes at a time over 32 slot residues, each access of a paired form like
-// a single one.
+// Slot layouts of one half's positions, 8-byte slots.  gfx950 serves ds_read_b64 32
+// lanes at a time over 32 slot residues, ds_write_b64 and each access of the
+// paired forms 16 lanes over 16.
 //  - Pad16, i + i/16: 17 slots per lane at M = 1 and 272 per 16 lanes at
 //    M = 16, both conflict free; a run of 32 consecutive positions (the
-//    M >= 64 passes) spans 33 slots and costs 2 cycles per access.
+//    M >= 64 passes) spans 33 slots, and a ds_read_b64 of it costs 2 cycles.
 //  - Pad256, i + 16*(i/256): 32-runs stay contiguous, and the M = 16 pass's
 //    two 16-runs per half-wavefront land 16 residues apart: conflict free for
 //    the passes at M >= 16, not at M = 1.

@@ -67,10 +67,11 @@ def conflict_cycles(slots, form: str) -> int:
 
 
 # ---- 4-byte forms ----------------------------------------------------------------
-# The N = 32768 conv (wide.hip) exchanges one float component at a time
-# (ds_read_b32 / ds_write_b32 and their paired and st64 forms).  Slots here
-# are float indices (byte address / 4).  Measured the same way as the 8-byte
-# forms (a one-off probe: one 64-lane workgroup per pattern and form, 256
+# ds_read_b32 / ds_write_b32 and their paired and st64 forms.  No kernel exchanges
+# its values with them now: the N = 32768 conv (wide.hip) did, one float component
+# at a time, before its rounds became halves of whole complex values.  Slots
+# here are float indices (byte address / 4).  Measured the same way as the
+# 8-byte forms (a one-off probe: one 64-lane workgroup per pattern and form, 256
 # repetitions, rocprofv3 --pmc SQ_LDS_BANK_CONFLICT SQ_INSTS_LDS SQ_WAVES):
 #
 # - every 4-byte form is serviced 32 lanes at a time over 32 banks; two lanes

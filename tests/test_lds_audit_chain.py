@@ -1,8 +1,8 @@
 """The LDS audit (test_lds_audit.py) for the plans of the four-step chain in one
 workgroup: a radix-16 outer level first, then the radix-16 plan of n / 16
-points, so the lead pass (radix 2, 4 or 8) is the second one.  N = 8192 and
-16384 at 16 values per lane with the per-exchange layouts, N = 32768 at 32
-values per lane with the float layouts."""
+points, so the lead pass (radix 2, 4 or 8) is the second one.  The exchanges of N =
+8192 and 16384 at 16 values per lane, with the per-exchange layouts; those of
+N = 32768 at 32 values per lane are in test_lds_audit_halves.py."""
 import pytest
 
 from tests import test_lds_audit as A
@@ -25,14 +25,6 @@ def chain_plan(n, v):
 def test_exchange_layouts(n, monkeypatch):
     monkeypatch.setattr(A, "plan", chain_plan)
     assert A.xchg_problems(n, 16, A.xchg_params) == []
-
-
-def test_wide_float_layouts(monkeypatch):
-    monkeypatch.setattr(A, "WIDE_RADICES", chain_radices(A.WIDE_N))
-    A.test_wide_private_exchange_rule_matches_brute_force()
-    A.test_wide_layouts_keep_wavefront_ranges()
-    A.test_wide_layouts_additive()
-    assert A._wide_conflicts(lambda p: A._pad16 if A._wide_private(p) else A._pad256) == 0
 
 
 @pytest.mark.parametrize("n,v,stride_lanes", [(8192, 16, 512), (16384, 16, 1024), (32768, 32, 1024)])

@@ -75,3 +75,19 @@ def test_conflict_free_and_additive(name):
                         s = [slot(n, x[g][k]) for x in lanes]
                         assert s == [b + slot(n, k * m) for b in base]
                         assert M.conflict_cycles(s, "read_b64") == 0 and M.conflict_cycles(s, "write_b64") == 0
+
+
+@pytest.mark.parametrize("name", PLANS)
+def test_private_exchange_rule_matches_brute_force(name):
+    """An exchange has wavefront fences in place of workgroup barriers where both
+    passes run at M <= 64 with the same radix: exactly where every wavefront reads
+    back, in each half, the positions that it wrote."""
+    n, radices = PLANS[name]
+    for p in range(len(radices) - 1):
+        private = True
+        for half in (0, 1):
+            for w in range(n // V // 64):
+                wrote, reads = ({x for lane in range(64 * w, 64 * w + 64) for g in taps(n, radices, q, lane, half)
+                                 for x in g} for q in (p, p + 1))
+                private &= wrote == reads
+        assert private == (stride(n, radices, p) <= 64 and radices[p] == radices[p + 1]), p

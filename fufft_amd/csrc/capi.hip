@@ -1061,30 +1061,6 @@ int fufft_plan_filter_large_device_f32(const void* in, void* out, int64_t n, int
    return run_conv1d(K_PLAN_TAPS, mn, v, p, stream);
 }
 
-// How many of a batch's four-step transforms run the whole chain in one
-// workgroup each (radix-16 middle, n <= 32768), reading and writing the data
-// once where the three launches do it three times; the rest run those.  The
-// results are the same bit for bit, so the line is the faster side.  A round of
-// up to 256 transforms (one per CU, where it holds no more) takes some 17 us at
-// n = 16384 and 33 at 32768, full or not, so a last round of a few is left to the
-// three launches.  us a call, shared filter, three buffers in turn, three launches
-// / one / split (whole rounds in one):
-//   n =  8192: 1 11.6 / 9.5, 64 12.4 / 10.1, 200 18.0 / 12.5, 400 32.8 / 18.6;
-//   n = 16384: 40 12.8 / 16.4, 64 14.8 / 16.7, 80 16.9 / 16.8, 128 20.2 / 17.5, 256
-//     36.6 / 21.8, 300 41.6 / 36.0 / 34.0, 340 47.2 / 37.3 / 38.3, 512 65.0 / 49.6;
-//   n = 32768: 100 29.2 / 35.6, 128 33.9 / 38.4, 160 42.9 / 40.8, 256 62.5 / 52.1, 301
-//     72.8 / 84.7 / 69.1, 384 92.5 / 88.9 / 86.2, 448 107 / 93 / 101, 530 125 / 132 /
-//     113, 768 181 / 149.
-// A filter per transform moves the lines little (n = 32768: 128 37.0 / 39.9, 160 46.7 /
-// 44.4, 384 109 / 95 / 94).
-static int64_t chain_batch(int64_t n, int v, int64_t batch)
-{
-   if(!conv_chain_plan(n, v)) return 0;
-   if(n == 8192) return batch;
-   const int64_t last = batch % 256;
-   return last >= (n == 16384 ? 80 : 144) ? batch : batch - last;
-}
-
 int fufft_conv_large_f32(void* buf, const void* filt, int64_t filt_stride, int64_t n,
                          int64_t batch, int mid, int variant, void* stream)
 {

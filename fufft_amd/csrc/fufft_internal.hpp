@@ -179,9 +179,36 @@ hipError_t launch_conv_wide(const Conv1dParams& p, int n, hipStream_t s);
 // The four-step chain of one outer level in one launch: K_CONV_CHAIN at
 // N = 8192 and 16384, the wide kernel at 32768.  Against the three launches:
 // 8192 x 4000 248.9 -> 124.8 us, 16384 x 300 43.4 -> 36.2, 32768 x 256 68.5 ->
-// 47.4; the batches that take it are chain_batch's choice (capi.hip).
+// 47.4; the batches that take it are chain_batch's choice.
 constexpr bool conv_chain_plan(int64_t n, int v) { return v == 16 && (n == 8192 || n == 16384 || n == CONV_WIDE_N); }
 hipError_t launch_conv_wide_chain(const Conv1dParams& p, int n, hipStream_t s);
+
+// How many of a batch's four-step transforms run the whole chain in one
+// workgroup each (radix-16 middle, n <= 32768), reading and writing the data
+// once where the three launches do it three times; the rest run those.  The
+// results are the same bit for bit, so the line is the faster side.  A round of
+// up to 256 transforms (one per CU, where it holds no more) takes 16 to 21 us at
+// n = 16384 and 28 to 48 at 32768, so a last round of a few is left to the three
+// launches.  us a call, shared filter, three buffers in turn, three launches / one
+// / split (whole rounds in one):
+//   n =  8192: 1 11.6 / 9.5, 64 12.4 / 10.1, 200 18.0 / 12.5, 400 32.8 / 18.6;
+//   n = 16384: 40 12.9 / 16.1, 64 14.6 / 16.0, 68 16.5 / 16.0, 80 16.9 / 16.0, 128 20.2
+//     / 17.1, 256 36.9 / 21.2, 300 42.0 / 34.8 / 34.3, 320 43.9 / 36.5 / 36.0, 328 46.2 /
+//     37.2 / 37.9, 512 66.0 / 49.3, 592 75.8 / 54.8 / 66.3;
+//   n = 32768: 1 11.6 / 28.5, 96 28.7 / 32.1, 112 31.7 / 32.9, 128 34.2 / 34.2, 132 36.7 /
+//     35.1, 144 40.6 / 35.9, 160 43.2 / 37.5, 256 63.8 / 47.7, 301 74.7 / 72.6 / 63.0, 352
+//     87.0 / 76.0 / 75.4, 368 90.7 / 77.0 / 78.1, 384 93.7 / 79.6 / 80.7, 448 110 / 82 / 96,
+//     530 129 / 115 / 102, 768 181 / 135.
+// A filter per transform moves the lines little (n = 32768: 112 33.7 / 34.0, 128 37.3 /
+// 36.3, 144 42.8 / 38.5, 352 101 / 80.7 / 79.8, 384 109 / 84 / 87; n = 16384: 64 14.6 / 16.3,
+// 68 16.6 / 16.4).
+constexpr int64_t chain_batch(int64_t n, int v, int64_t batch)
+{
+   if(!conv_chain_plan(n, v)) return 0;
+   if(n == 8192) return batch;
+   const int64_t last = batch % 256;
+   return last >= (n == 16384 ? 68 : 128) ? batch : batch - last;
+}
 
 // ---- filter planning on the device (plan.hip) ----------------------------------------
 struct GatherDigits {

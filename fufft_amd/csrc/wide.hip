@@ -45,7 +45,7 @@
 // in that order, for a filter in the chain order: one read and one write of the
 // data where fufft_conv_large_f32's three launches make three of each.  1000
 // transforms 244 us in three launches, 174 here; which batches take it is
-// chain_batch's choice (capi.hip).
+// chain_batch's choice (fufft_internal.hpp).
 //
 // N = 16384 runs the same code with 512 lanes (LEAD 4, eight groups per lane
 // in the lead pass): 68 KiB of LDS, so two workgroups share a CU and one's

@@ -109,9 +109,10 @@ def test_large_rejects_bad_args(dev):
 
 
 @pytest.mark.parametrize("own_filters", [False, True])
-@pytest.mark.parametrize("n,batch", [(8192, 1), (8192, 257), (16384, 79), (16384, 80), (16384, 335), (16384, 336),
-                                     (32768, 143), (32768, 144), (32768, 256), (32768, 257), (32768, 399),
-                                     (32768, 400)])
+@pytest.mark.parametrize("n,batch", [(8192, 1), (8192, 257), (16384, 67), (16384, 68), (16384, 79), (16384, 80),
+                                     (16384, 323), (16384, 324), (16384, 335), (16384, 336), (32768, 127),
+                                     (32768, 128), (32768, 143), (32768, 144), (32768, 256), (32768, 257), (32768, 383),
+                                     (32768, 384), (32768, 399), (32768, 400)])
 def test_large_split_between_one_launch_and_three(dev, n, batch, own_filters):
     """Up to n = 32768 the batch decides how many transforms run the chain in one
     workgroup and how many in three launches.  On both sides of every line the

@@ -457,3 +457,52 @@ int main() { return 0; }
                         f"-I{ROOT / 'include'}", f"-I{ROOT / 'fufft_amd' / 'csrc'}", f"-I{rocm / 'include'}", str(src)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+# us a call of fufft_conv_large_f32, shared filter, three buffers in turn: three
+# launches, one, whole rounds in one and the last in three
+CHAIN_US = {
+    16384: {40: (12.87, 16.07, 12.84), 64: (14.58, 16.01, 14.60), 72: (16.67, 16.01, 16.70), 96: (17.54, 16.59, 17.52),
+            128: (20.15, 17.07, 20.05), 256: (36.89, 21.19, 21.18), 312: (43.12, 36.33, 35.19), 328: (46.15, 37.17, 37.92),
+            592: (75.80, 54.76, 66.26)},
+    32768: {88: (27.45, 31.74, 27.45), 112: (31.67, 32.91, 31.65), 120: (32.83, 33.60, 32.84), 136: (37.63, 34.93, 37.55),
+            140: (39.93, 35.71, 40.02), 160: (43.18, 37.53, 43.29), 256: (63.76, 47.70, 47.83), 336: (82.13, 75.85, 72.29),
+            384: (93.66, 79.55, 80.72), 400: (97.38, 79.01, 86.10), 624: (150.07, 122.68, 123.94), 656: (157.18, 124.01, 133.08)},
+}
+
+
+def test_four_step_rule_takes_the_faster_side(tmp_path):
+    """chain_batch, compiled: within 2% of the fastest measured way for every
+    batch of the table; all of a batch at n = 8192, none with the radix-8 middle
+    or beyond 32768; never more than the batch."""
+    import shutil
+    import subprocess
+    rocm = Path("/opt/rocm")
+    if shutil.which("g++") is None or not (rocm / "include" / "hip" / "hip_runtime.h").exists():
+        pytest.skip("g++ or the HIP headers are not available")
+    src, exe = tmp_path / "chain.cpp", tmp_path / "chain"
+    src.write_text('''
+#include "fufft_internal.hpp"
+#include <cstdio>
+int main()
+{
+   for(int64_t n = 8192; n <= 65536; n *= 2)
+      for(int v : {8, 16})
+         for(int64_t b = 0; b < 1200; b++)
+            std::printf("%lld %d %lld %lld\\n", (long long)n, v, (long long)b, (long long)fufft::chain_batch(n, v, b));
+}
+''')
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{ROOT / 'include'}",
+                    f"-I{ROOT / 'fufft_amd' / 'csrc'}", f"-I{rocm / 'include'}", str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    rule = {tuple(map(int, line.split()[:3])): int(line.split()[3]) for line in out.splitlines()}
+    assert len(rule) == 4 * 2 * 1200
+    for (n, v, b), whole in rule.items():
+        assert 0 <= whole <= b
+        assert whole in ((0,) if v == 8 or n > 32768 else (b,) if n == 8192 else (b, b - b % 256))
+    for n, rows in CHAIN_US.items():
+        for b, us in rows.items():
+            three, one, split = us
+            whole = rule[n, 16, b]
+            taken = one if whole == b else split if whole else three
+            assert taken <= 1.02 * min(us), (n, b, taken, us)

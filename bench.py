@@ -374,6 +374,16 @@ def bench_r2(torch, ff, dev, n, pts, steps, warmup, stream, seed):
             "rel_l2": rel}
 
 
+def one_launch_transforms(n: int, batch: int, variant: str) -> int:
+    """How many transforms of a four-step batch fufft_conv_large_f32 runs whole in
+    one launch (chain_batch in fufft_amd/csrc/fufft_internal.hpp); the others take
+    its three launches."""
+    if variant != "v16" or n not in (8192, 16384, 32768):
+        return 0
+    last = batch % 256
+    return batch if n == 8192 or last >= (68 if n == 16384 else 128) else batch - last
+
+
 def bench_large(torch, ff, dev, n, pts, steps, warmup, stream, seed, variant="auto", per_transform=False):
     """Four-step conv: batch pts/n of U[-1,1) signals, one
     shared filter in the chain order of the middle `variant` ("auto" = "v16",
@@ -1015,12 +1025,17 @@ def main():
                 print(json.dumps({"error": f"four-step accuracy check failed at N={s} ({lv}): rel L2 {r:.3e}"}))
                 sys.exit(1)
             model = (4 * lout + 3) * 8
+            # one read and one write of 8 B where the whole chain runs in one
+            # launch; else three passes of 16 B (the two outer levels of a
+            # two-level plan run as one pass); the filter is cache-resident
+            batch = pts // s
+            whole = one_launch_transforms(s, batch, lv)
+            moved = 16.0 * whole / batch + 48.0 * (batch - whole) / batch
             legs[lv] = {"gpoints_s": round(pts / a / 1e9, 3), "ms": round(a * 1e3, 5),
                         "plan": f"{lout} outer radix-16 level(s) + fused middle N={mid} at "
-                                f"{'radix 16 (the reference run_large middle)' if lv == 'v16' else 'radix 8'}",
-                        # three passes of 16 B (the two outer levels of a two-level plan
-                        # run as one pass); the filter is cache-resident
-                        "bytes_per_point": 48, "frac": frac(48.0 * pts, a),
+                                f"{'radix 16 (the reference run_large middle)' if lv == 'v16' else 'radix 8'}; "
+                                f"{whole} of {batch} transforms whole in one launch, the others in three",
+                        "bytes_per_point": round(moved, 2), "frac": frac(moved * pts, a),
                         # the reference's (4 lout + 3) x 8 B model (bench_fufft.cu:481)
                         "model_bytes_per_point": model,
                         "model_frac": round(model * pts / a / 1e9 / HBM_PEAK_GBS, 4),
@@ -1029,8 +1044,8 @@ def main():
         large[str(s)] = {**legs["v16"], "variant": "v16", "r8_middle": legs["r8"]}
         if not args.no_per_signal:
             # the reference's own run_large protocol: one chained filter per
-            # transform, a fourth 8 B/pt stream (its 56 B/pt model is then the
-            # physical bytes)
+            # transform, 8 B/pt more (in three launches its 56 B/pt model is then
+            # the physical bytes)
             a, r = bench_large(torch, ff, dev, s, pts, args.sweep_steps, 3, stream, 7 + s, variant="v16",
                                per_transform=True)
             if not r <= 2e-6:
@@ -1039,8 +1054,9 @@ def main():
                 sys.exit(1)
             large[str(s)]["per_transform_filter"] = {
                 "what": "one chained filter per transform, as the reference's run_large (fufft::ref::run_large)",
-                "gpoints_s": round(pts / a / 1e9, 3), "ms": round(a * 1e3, 5), "bytes_per_point": 56,
-                "frac": frac(56.0 * pts, a), "rel_l2": r}
+                "gpoints_s": round(pts / a / 1e9, 3), "ms": round(a * 1e3, 5),
+                "bytes_per_point": legs["v16"]["bytes_per_point"] + 8,
+                "frac": frac((legs["v16"]["bytes_per_point"] + 8) * pts, a), "rel_l2": r}
         if not args.no_vendor:
             # the reference times its four-step against the cuFFT chain at this N
             # (bench_fufft.cu:453-478); here rocFFT through torch.fft, same batch

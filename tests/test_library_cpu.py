@@ -506,3 +506,7 @@ int main()
             whole = rule[n, 16, b]
             taken = one if whole == b else split if whole else three
             assert taken <= 1.02 * min(us), (n, b, taken, us)
+    # the benchmark charges each transform the bytes of the way it takes
+    import bench
+    for (n, v, b), whole in rule.items():
+        assert bench.one_launch_transforms(n, b, "v16" if v == 16 else "r8") == whole

@@ -576,7 +576,7 @@ int fufft_conv_f32(const void* in, const void* filt, int64_t filt_stride,
    const int kind = per_signal && layout == FUFFT_LAYOUT_LANE &&
                     (conv_psf_plan((int)n, v) || conv_psf_late_plan((int)n, v))             ? K_CONV_PSF
                   : per_signal && layout == FUFFT_LAYOUT_DR && conv_psf_dr_plan((int)n, v) ? K_CONV_PSF_DR
-                  : conv_near(n, batch) && lds_layout() != LAYOUT_XOR                      ? K_CONV_NEAR
+                  : conv_near(n, batch, per_signal) && lds_layout() != LAYOUT_XOR          ? K_CONV_NEAR
                                                                                            : K_CONV;
    return run_conv1d(kind, (int)n, v, p, stream);
 }
@@ -698,7 +698,8 @@ int fufft_c2c_f32(const void* in, void* out, int64_t n, int64_t batch, int direc
    if((st = current_table(&p.tw)) != FUFFT_OK) return st;
    p.in0 = in; p.out0 = out; p.ntrans = (uint32_t)batch;
    p.fcount = 1; p.scount = 1; p.mid = FUFFT_MID_NONE; p.fl = FUFFT_LAYOUT_DR;
-   const int kind = direction == FUFFT_INVERSE ? K_C2C_INV : c2c_far(n, batch) ? K_C2C_FAR : K_C2C_FWD;
+   const bool far = c2c_far(n, batch) && lds_layout() != LAYOUT_XOR;
+   const int kind = direction == FUFFT_FORWARD ? (far ? K_C2C_FAR : K_C2C_FWD) : (far ? K_C2C_INV_FAR : K_C2C_INV);
    return run_conv1d(kind, (int)n, v, p, stream);
 }
 

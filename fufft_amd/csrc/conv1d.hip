@@ -37,7 +37,7 @@ constexpr int cpb_for(int T) { return T >= 128 ? 1 : 256 / T; }
 // (the forward's pass-0 scatter) are the same positions of the same layout,
 // which no other lane touches in between.
 template<int N, int KIND>
-constexpr bool conv_loops() { return (KIND == K_CONV || KIND == K_CONV_CHAIN) && N == 16384; }
+constexpr bool conv_loops() { return (KIND == K_CONV || KIND == K_CONV_NEAR || KIND == K_CONV_CHAIN) && N == 16384; }
 
 // The count is the launch's choice: a CU runs ceil(workgroups / CUs) of them
 // one after the other, iters transforms each, so the launch takes the iters
@@ -94,7 +94,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    constexpr bool FROM_SPEC = KIND == K_APPLY || FROM_ROWS;
    constexpr bool TO_SPEC   = KIND == K_FWD || KIND == K_FWD_ROWS || KIND == K_FWD_R2;
    constexpr bool C2C_FWD   = KIND == K_C2C_FWD || KIND == K_C2C_FAR;
-   constexpr bool C2C_INV   = KIND == K_C2C_INV;
+   constexpr bool C2C_INV   = KIND == K_C2C_INV || KIND == K_C2C_INV_FAR;
    constexpr bool PLAN      = KIND == K_PLAN_TAPS;
    constexpr bool TIMED     = KIND == K_CONV_TIMED;
    // one filter per signal: its loads go out with the signal's (lane-major
@@ -106,26 +106,26 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // the mid as usual, streamed past the caches
    constexpr bool PSF_LATE  = PSF_ANY && !PSF;
    // Cache policy of the signal's loads and the result's stores (figures at
-   // POL_WT in fufft_device.hpp and conv_near in fufft_internal.hpp).  What the
-   // program's or the path's next launch reads -- 2D rows, the four-step middle,
-   // a C2C spectrum on its way back -- is written through (WT); the other results
-   // stream past the caches (NT), which leaves these to what is read, except at
-   // N = 16384, where writing through measured 2-10% faster (8 M points 52.0 -> 46.4
-   // us).  The loads stream too where the signals are more than the last-level
-   // cache keeps.  The split forward keeps the default: its digit-order stores
-   // are 16-byte pieces that the L2 puts together.  So does the real conv at N =
-   // 256, whose 16 lanes store 64 bytes, half a line (us, default / streamed, real
-   // pairs in turn: one of 16 M points 43.9 / 49.0, three 53.2 / 56.2; 134 M 386 / 403).
+   // POL_WT in fufft_device.hpp, conv_near and c2c_far in fufft_internal.hpp).  What
+   // the program's or the path's next launch reads -- 2D rows, the four-step middle,
+   // C2C results and those of the N = 16384 conv, as long as the last-level cache
+   // holds them -- is written through (WT); the other results stream past the caches
+   // (NT), which leaves these to what is read.  The loads stream too where the
+   // signals are more than the cache keeps.  The split forward keeps the default:
+   // its digit-order stores are 16-byte pieces that the L2 puts together.  So does
+   // the real conv at N = 256, whose 16 lanes store 64 bytes, half a line (us, default
+   // / streamed, real pairs in turn: one of 16 M points 43.9 / 49.0, three 53.2 / 56.2;
+   // 134 M 386 / 403).
    constexpr int  EL_IN  = REAL_IN ? 4 : 8;
    constexpr int  EL_OUT = REAL_OUT ? 4 : 8;
    constexpr bool LINES = (T < 64 ? T : 64) * EL_OUT >= 128;   // a wavefront's store covers whole lines
+   constexpr bool NEAR_ST = KIND == K_CONV_NEAR && N == 16384, NEAR_LD = KIND == K_CONV_NEAR && !NEAR_ST;
    constexpr bool ONCE = KIND == K_CONV || KIND == K_CONV_PSF || KIND == K_CONV_PSF_DR || CHAIN || TIMED;
    constexpr bool KEPT = KIND == K_CONV_MID || KIND == K_FWD_ROWS || KIND == K_FWD_R2 || KIND == K_APPLY_ROWS ||
-                         KIND == K_APPLY_R2 || KIND == K_C2C_FWD || C2C_INV ||
-                         ((KIND == K_CONV || TIMED) && N == 16384);
-   constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV) ? POL_NT : POL_DEFAULT;
+                         KIND == K_APPLY_R2 || KIND == K_C2C_FWD || KIND == K_C2C_INV || NEAR_ST;
+   constexpr int  LD_POL = (ONCE || C2C_FWD || C2C_INV || NEAR_ST) ? POL_NT : POL_DEFAULT;
    constexpr int  ST_POL = KEPT ? POL_WT
-                         : (ONCE || KIND == K_C2C_FAR || KIND == K_CONV_NEAR || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY)
+                         : (ONCE || C2C_FWD || C2C_INV || NEAR_LD || (KIND == K_CONV_R2 && LINES) || KIND == K_APPLY)
                               ? POL_NT : POL_DEFAULT;
 
    extern __shared__ float2 lds[];
@@ -144,6 +144,9 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
    // workgroup arrived, then the shader clock (reads only; thread 0 writes the
    // record with ordinary vector stores at the end)
    uint64_t ts[TIMER_MARKS + 1], rt0 = 0;
+   // the timer reads and writes as the conv of this batch does, K_CONV_NEAR or K_CONV
+   bool near = false;
+   if constexpr(TIMED) near = conv_near(N, p.ntrans, p.fcount > 1);
    auto stamp = [&](int i) {
       if constexpr(TIMED) {
          __builtin_amdgcn_s_waitcnt(0);
@@ -215,10 +218,7 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
             r[q] = make_float2(xb.ld1<LD_POL>(lane_pos * 4u, q * T * 4), yb.ld1<LD_POL>(lane_pos * 4u, q * T * 4));
       } else {
          const Buf xb(static_cast<const char*>(p.in0) + wb, WB);
-         // the timer reads as the conv of this batch does, K_CONV_NEAR or K_CONV
-         bool near = false;
-         if constexpr(TIMED) near = conv_near(N, p.ntrans);
-         if(TIMED && near) {
+         if(TIMED && N <= 8192 && near) {
 #pragma unroll
             for(int q = 0; q < V; q++) r[q] = xb.ld2(lane_pos * 8u, q * T * 8);
          } else {
@@ -325,8 +325,13 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
          }
       } else {
          const Buf ob(static_cast<char*>(p.out0) + wb, WB);
+         if(TIMED && N == 16384 && near) {
 #pragma unroll
-         for(int q = 0; q < V; q++) ob.st2<ST_POL>(r[q], lane_pos * 8u, q * T * 8);
+            for(int q = 0; q < V; q++) ob.st2<POL_WT>(r[q], lane_pos * 8u, q * T * 8);
+         } else {
+#pragma unroll
+            for(int q = 0; q < V; q++) ob.st2<ST_POL>(r[q], lane_pos * 8u, q * T * 8);
+         }
       }
       if constexpr(TIMED) {
          stamp(5);
@@ -360,14 +365,14 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
 // straight: the split apply (a spectrum and a filter per transform, N = 1024 570
 // / 604; one spectrum, N = 4096 373 / 387) and the near conv (N = 1024, 8 M points
 // 23.65 / 23.95).
-template<int KIND>
-constexpr bool conv_straight() { return KIND == K_APPLY || KIND == K_CONV_NEAR; }
+template<int N, int KIND>
+constexpr bool conv_straight() { return KIND == K_APPLY || (KIND == K_CONV_NEAR && !conv_loops<N, KIND>()); }
 
 template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_straight<KIND>()) {
+   if constexpr(conv_straight<N, KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x);
    } else {
       const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
@@ -382,7 +387,7 @@ template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_bperm_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_straight<KIND>()) {
+   if constexpr(conv_straight<N, KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x);
    } else {
       const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
@@ -480,8 +485,11 @@ static hipError_t launch_kind(int kind, const Conv1dParams& p, hipStream_t s)
                                   : hipErrorInvalidValue;
       case K_C2C_FWD:   return launch_one<N, V, LAYOUT, K_C2C_FWD, MID_NONE>(p, s);
       case K_C2C_FAR:
-         if constexpr(c2c_far_plan(N)) return launch_one<N, V, LAYOUT, K_C2C_FAR, MID_NONE>(p, s);
-         else                          return hipErrorInvalidValue;
+         if constexpr(LAYOUT != LAYOUT_XOR) return launch_one<N, V, LAYOUT, K_C2C_FAR, MID_NONE>(p, s);
+         else                               return hipErrorInvalidValue;
+      case K_C2C_INV_FAR:
+         if constexpr(LAYOUT != LAYOUT_XOR) return launch_one<N, V, LAYOUT, K_C2C_INV_FAR, MID_NONE>(p, s);
+         else                               return hipErrorInvalidValue;
       case K_C2C_INV:   return launch_one<N, V, LAYOUT, K_C2C_INV, MID_NONE>(p, s);
       case K_PLAN_TAPS: return launch_one<N, V, LAYOUT, K_PLAN_TAPS, MID_NONE>(p, s);
       case K_CONV_TIMED:

@@ -280,7 +280,8 @@ __device__ __forceinline__ void twiddle_group(float2 (&r)[NR], float2 w1)
 // the next launch reads, us, default -> WT: four-step 32768 x 50 28.2 -> 18.1, x 301
 // 78.4 -> 74.1, 65536 x 16 22.7 -> 16.3, x 500 247 -> 244, 2^20 x 1 24.9 -> 18.4, x 3 35.9 ->
 // 31.5; conv 2D 256 x 1024 x 8 28.9 -> 25.5, 512 x 512 x 4 19.0 -> 17.3, x 64 137.9 -> 133.0;
-// C2C both ways N = 4096, 2 M points 18.2 -> 14.8, 8 M 46.5 -> 44.2, 17 M 89.1 -> 86.8.
+// C2C both ways N = 4096, 2 M points 18.2 -> 14.8, 8 M 46.5 -> 44.2, 17 M 89.1 -> 86.8
+// (results that the last-level cache cannot hold are streamed, c2c_far).
 // For results nothing reads next NT stays: conv N = 1024, 8 M points 24.0, WT 31.4.
 enum { POL_DEFAULT = 0, POL_NT = 2, POL_WT = 16 };
 

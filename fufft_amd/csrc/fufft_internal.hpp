@@ -46,8 +46,9 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 // K_FWD / K_APPLY: the split forward and apply, spectra in digit order;
 // K_FWD_ROWS / K_APPLY_ROWS: the row forward and inverse of the 2D paths,
 // lane-major spectra and no mid operation.
-// K_CONV_NEAR: K_CONV for signals that the last-level cache keeps: default
-// loads (conv_near).  K_C2C_FAR: K_C2C_FWD with streamed stores (c2c_far).
+// K_CONV_NEAR: K_CONV for signals (at N = 16384: results) that the last-level cache
+// keeps: default loads (written through; conv_near).  K_C2C_FAR, K_C2C_INV_FAR: the
+// C2C with streamed stores (c2c_far).
 // K_FWD_R2 / K_APPLY_R2: the forward half reading two real arrays, the
 // inverse half writing two real arrays (2D two-for-one rows).
 // K_C2C_FWD / K_C2C_INV: natural order in and out (forward DIF + digit ->
@@ -72,7 +73,8 @@ __host__ __device__ constexpr uint32_t lane_position(uint32_t slot, uint32_t tlo
 enum { K_CONV = 0, K_CONV_R2 = 1, K_FWD = 2, K_APPLY = 3, K_FWD_R2 = 4, K_APPLY_R2 = 5,
        K_C2C_FWD = 6, K_C2C_INV = 7, K_PLAN_TAPS = 8, K_CONV_TIMED = 9, K_CONV_MID = 10,
        K_CONV_PSF = 11, K_CONV_PSF_DR = 12, K_CONV_CHAIN = 13,
-       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_FWD_ROWS = 16, K_C2C_FAR = 17 };
+       K_CONV_NEAR = 14, K_APPLY_ROWS = 15, K_FWD_ROWS = 16, K_C2C_FAR = 17,
+       K_C2C_INV_FAR = 18 };
 
 // the plans K_CONV_PSF and K_CONV_PSF_DR are built for: radix 16 with whole
 // wavefronts per transform and room for the filter's 32 VGPRs within 128
@@ -92,7 +94,7 @@ constexpr bool conv_psf_dr_plan(int n, int v) { return v == 16 && (n == 2048 || 
 // 213.3, so those sizes keep the plain kernel.
 constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 
-// K_CONV_NEAR runs the conv whose signals take up to 80 MiB of the 256 MiB
+// K_CONV_NEAR, N <= 8192: the conv whose signals take up to 80 MiB of the 256 MiB
 // last-level cache.  What a program convolves was mostly just written, or is
 // convolved again, and a default load keeps it there, where a streaming one
 // has the next pass fetch it from HBM.  Three states in turn, us, loads and
@@ -108,28 +110,37 @@ constexpr bool conv_psf_late_plan(int n, int v) { return v == 8 && n == 512; }
 // Sixteen of 64 MiB in turn 29.0 / 29.4.  Signals that come from HBM to a cache
 // full of results push those out under the conv: with 1 GiB written before each
 // call, both together, 64 MiB 185 / 192, 120 MiB 204 / 220; with 128 MiB 49.5 / 44.8.
+//
+// K_CONV_NEAR, N = 16384: the conv whose result, with the filters where each signal
+// has its own, takes up to the 256 MiB; it streams its loads and writes its
+// results through.  us, streamed / written through: 1.6 M points 17.6 / 17.3, 6 M
+// 40.9 / 39.8, 12 M 63.6 / 61.4, 24 M 120 / 117, 32 M 156 / 155 (three buffers in
+// turn; in place 32 M 157 / 135), with a scaling of the result behind it 8 M 77.7
+// / 75.4, 32 M 236 / 223, but 64 M 461 / 506, 134 M 936 / 991; a filter per signal
+// 12 M 63.3 / 59.4, 16 M 82.7 / 78.1, 24 M 120 / 128, 32 M 156 / 165.  Even or slower
+// by up to 6%: 8 M in turn, 48.9 / 52.0.
+//
 // The other single-launch kinds have one policy.  Stores streamed, loads not:
 // the split apply (N = 512 / 4096 / 8192, 8 M points 29.3 / 33.6 / 38.9 -> 24.3 / 26.9
 // / 31.5, 34 M 97 / 104 / 118 -> 94 / 102 / 115), the real conv from N = 512 on (8 M,
 // N = 4096 31.9 -> 26.5) and the small images but 8 x 64 and 16 x 64; both streamed:
-// one filter per signal, the four-step chain and N >= 16384, which measured best
-// or even so.
-constexpr bool conv_near_plan(int64_t n) { return n <= 8192; }
-constexpr bool conv_near(int64_t n, int64_t batch)
+// one filter per signal at N <= 4096, the four-step chain and N = 32768, which
+// measured best or even so.
+constexpr bool conv_near_plan(int64_t n) { return n <= 16384; }
+constexpr bool conv_near(int64_t n, int64_t batch, bool per_signal)
 {
-   return conv_near_plan(n) && batch <= ((int64_t)80 << 20) / (8 * n);
+   if(n <= 8192) return batch <= ((int64_t)80 << 20) / (8 * n);
+   return n == 16384 && batch <= ((int64_t)(per_signal ? 128 : 256) << 20) / (8 * n);
 }
 
-// K_C2C_FAR: spectra of more than 512 MiB at N = 256.  Nothing of them is in the
-// caches when the next launch reads it, and at this size alone streaming is then
-// the faster.  us, written through / streamed: 67 M points 173 / 173, 84 M 221.5 /
-// 218, 101 M 270 / 264, 134 M 369 / 357; N = 1024, 134 M 344 / 349; N = 4096 and the
-// inverses even or faster written through.
-constexpr bool c2c_far_plan(int64_t n) { return n == 256; }
-constexpr bool c2c_far(int64_t n, int64_t batch)
-{
-   return c2c_far_plan(n) && batch > ((int64_t)512 << 20) / (8 * n);
-}
+// K_C2C_FAR, K_C2C_INV_FAR: results of more than the 256 MiB, streamed.  Nothing of
+// them is in the cache when the next launch reads it, and written through they
+// leave the cache full of lines that the next launch has to push out.  us, written
+// through / streamed, with a scaling of the result behind: N = 4096, 8 M points 47
+// / 55, 32 M 156 / 171, 42 M 227 / 210, 50 M 279 / 251, 67 M 367 / 333, 134 M 740 / 705;
+// N = 256 42 M 224 / 210; N = 16384 67 M 430 / 406.  A forward and its inverse 8 M 43
+// / 49, 34 M at N = 1024 even, 67 M 337 / 341; alone, N = 256 134 M 363 / 355.
+constexpr bool c2c_far(int64_t n, int64_t batch) { return batch > ((int64_t)256 << 20) / (8 * n); }
 
 // phase timer record of one workgroup (K_CONV_TIMED), TIMER_STRIDE words:
 // [0] HW_ID, [1] XCC_ID, [2] marks, [3] s_memrealtime ticks (100 MHz) from

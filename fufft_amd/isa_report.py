@@ -43,7 +43,7 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 KINDS = {0: "conv", 1: "conv_r2", 2: "fwd", 3: "apply", 4: "fwd_r2", 5: "apply_r2",
          6: "c2c_fwd", 7: "c2c_inv", 8: "plan_taps", 9: "conv_timed", 10: "conv_mid",
          11: "conv_psf", 12: "conv_psf_dr", 13: "conv_chain", 14: "conv_near", 15: "apply_rows",
-         16: "fwd_rows", 17: "c2c_far"}
+         16: "fwd_rows", 17: "c2c_far", 18: "c2c_inv_far"}
 MIDS = {0: "mul", 1: "conj", 2: "none"}
 LAYOUTS = {0: "xor", 1: "pad", 2: "xchg"}
 FILTERS = {0: "dr", 1: "lane", 2: "bperm"}
@@ -217,8 +217,8 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
         kind, mid = "apply", "none"
     if kind == "fwd_rows":
         kind = "fwd"
-    if kind == "c2c_far":
-        kind = "c2c_fwd"
+    if kind in ("c2c_far", "c2c_inv_far"):
+        kind = "c2c_fwd" if kind == "c2c_far" else "c2c_inv"
     ps = plan(n, v, chain)
     one_dir = sum(pass_ops(v, r, M, n // v) for r, M in ps)
     exchanges = len(ps) - 1
@@ -261,7 +261,8 @@ def model_conv(n: int, v: int, kind: str = "conv", mid: str = "mul") -> dict:
     untaken_loads = v // 2 if (kind in ("conv", "conv_r2", "conv_timed", "apply", "apply_r2") and mid != "none") else 0
     if kind == "conv_timed" and n <= 8192:
         untaken_loads += v               # the signal read with the other cache policy (conv_near)
-    untaken = {"loads": untaken_loads, "stores": v if kind == "plan_taps" else 0}
+    two_stores = kind == "plan_taps" or (kind == "conv_timed" and n == 16384)
+    untaken = {"loads": untaken_loads, "stores": v if two_stores else 0}
     return {"fp32_arith_per_lane": arith, "lds_access_8B_per_lane": lds, "vmem_loads_per_wave": loads,
             "vmem_stores_per_wave": stores, "untaken_branch": untaken, "passes": ps}
 

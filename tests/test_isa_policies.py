@@ -51,29 +51,35 @@ def test_real_conv_streams_whole_lines_only(conv1d, n, v, policy):
 
 
 @pytest.mark.parametrize("n,v", [(256, 16), (512, 8), (1024, 16), (4096, 8), (4096, 16), (16384, 16)])
-def test_c2c_spectra_are_written_through(conv1d, n, v):
-    """What the inverse reads back is written through; at N = 256 the forward has
-    a kernel that streams, for spectra of more than 512 MiB."""
-    assert stores(conv1d[kernel(n, v, 6, mid=2)]) == {"sc1"}
-    assert stores(conv1d[kernel(n, v, 7, mid=2)]) == {"sc1"}
-    far = kernel(n, v, 17, mid=2)
-    assert (stores(conv1d[far]) == {"nt"}) if n == 256 else (far not in conv1d)
+def test_c2c_results(conv1d, n, v):
+    """Written through for the launch that reads them next, with kernels that
+    stream for results the last-level cache cannot hold."""
+    for kind, far in ((6, 17), (7, 18)):
+        assert stores(conv1d[kernel(n, v, kind, mid=2)]) == {"sc1"}
+        assert stores(conv1d[kernel(n, v, far, mid=2)]) == {"nt"}
+
+
+def test_n16384_conv_results(conv1d):
+    """As the C2C's; the signals are streamed in both."""
+    for kind, policy in ((0, "nt"), (14, "sc1")):
+        got = conv1d[kernel(16384, 16, kind)]
+        assert stores(got) == {policy}
+        assert sum(p == "nt" for op, p in got if op == "buffer_load_dwordx2") == 16
 
 
 @pytest.mark.parametrize("n,v", [(256, 16), (512, 8), (1024, 16), (4096, 16), (4096, 8), (8192, 8), (16384, 16)])
 def test_phase_timer_has_the_policies_of_the_conv(conv1d, n, v):
-    """The timed kernel stores as the conv of the same plan does, and where that
-    has a kernel with default loads for small batches, it holds both reads."""
+    """The timed kernel holds the loads and stores of both convs of the plan, the one
+    for batches that the caches keep (K_CONV_NEAR) and the one for the others."""
     layout = 1 if (n, v) == (8192, 8) else 2
-    conv, timed = (conv1d[kernel(n, v, k, layout=layout)] for k in (0, 9))
-    assert stores(timed, "dwordx2") == stores(conv, "dwordx2") == ({"sc1"} if n == 16384 else {"nt"})
-    near = kernel(n, v, 14, layout=layout)
-    assert (near in conv1d) == (n <= 8192)
-    streamed = sum(p == "nt" for op, p in timed if op == "buffer_load_dwordx2")
-    default = sum(p == "default" for op, p in timed if op == "buffer_load_dwordx2")
-    plain = sum(p == "default" for op, p in conv if op == "buffer_load_dwordx2")
-    assert streamed == v
-    assert default == plain + (v if n <= 8192 else 0)
+    conv, near, timed = (conv1d[kernel(n, v, k, layout=layout)] for k in (0, 14, 9))
+    assert stores(timed, "dwordx2") == stores(conv, "dwordx2") | stores(near, "dwordx2")
+    plain = sum(p == "default" for op, p in conv if op == "buffer_load_dwordx2")       # the twiddles
+    for policy in ("nt", "default"):
+        of = [sum(p == policy for op, p in k if op == "buffer_load_dwordx2") for k in (conv, near, timed)]
+        assert of[2] == max(of[:2]), policy
+    assert {sum(p == "default" for op, p in k if op == "buffer_load_dwordx2") for k in (conv, near)} == \
+        ({plain} if n == 16384 else {plain, plain + v})
 
 
 @pytest.mark.parametrize("h,w,policy", [(8, 64, "default"), (16, 64, "default"), (32, 64, "nt"), (64, 64, "nt"),

@@ -433,11 +433,12 @@ def test_cpp_plan_objects_build_and_reject_bad_arguments(tmp_path):
     assert out.stdout.startswith("ok")
 
 
-def test_near_conv_leaves_room_for_the_next_batches(tmp_path):
-    """The rule that gives a conv default loads (conv_near) holds only where
-    three batches of its signals fit the 256 MiB last-level cache together: a
-    program that convolves them in turn otherwise has each one pushed out
-    before it comes back.  No batch size of N >= 16384 takes it."""
+def test_cache_rules_leave_room(tmp_path):
+    """The rules on what stays in the 256 MiB last-level cache.  Default loads of the
+    conv up to N = 8192: only where three batches of its signals fit together (a
+    program that convolves them in turn otherwise has each one pushed out before it
+    comes back).  Results written through, N = 16384 and the C2C: only where the
+    result fits, with the filters where each signal has its own."""
     import shutil
     import subprocess
     rocm = Path("/opt/rocm")
@@ -446,14 +447,20 @@ def test_near_conv_leaves_room_for_the_next_batches(tmp_path):
     src = tmp_path / "near.cpp"
     src.write_text('''
 #include "fufft_internal.hpp"
-constexpr int64_t most(int64_t n) { int64_t b = 0; while(fufft::conv_near(n, b + 1)) b++; return b; }
-constexpr bool fits(int64_t n) { return most(n) > 0 && 3 * most(n) * n * 8 <= (int64_t)256 << 20; }
-static_assert(fits(2048) && fits(4096) && fits(8192), "three batches in the cache");
-static_assert(!fufft::conv_near(256, (88 << 20) / (8 * 256)) && !fufft::conv_near(512, (96 << 20) / (8 * 512)), "");
-static_assert(most(16384) == 0 && most(32768) == 0, "one policy");
+constexpr int64_t LLC = (int64_t)256 << 20;
+constexpr int64_t most(int64_t n, bool own) { int64_t b = 0; while(fufft::conv_near(n, b + 1, own)) b++; return b; }
+constexpr int64_t kept(int64_t n) { int64_t b = 0; while(!fufft::c2c_far(n, b + 1)) b++; return b; }
+constexpr bool fits(int64_t n, bool own) { return most(n, own) > 0 && 3 * most(n, own) * n * 8 <= LLC; }
+static_assert(fits(2048, false) && fits(4096, false) && fits(8192, false) && fits(8192, true), "three batches");
+static_assert(!fufft::conv_near(256, (88 << 20) / (8 * 256), false) && !fufft::conv_near(512, (96 << 20) / (8 * 512), true), "");
+static_assert(most(16384, false) * 16384 * 8 == LLC && most(16384, true) * 16384 * 8 * 2 == LLC, "the result, the filters");
+static_assert(most(32768, false) == 0 && most(32768, true) == 0, "one policy");
+static_assert(kept(16384) * 16384 * 8 == LLC && kept(4096) * 4096 * 8 == LLC && kept(2048) * 2048 * 8 == LLC, "the result");
+static_assert(!fufft::c2c_far(256, LLC / 2048) && fufft::c2c_far(256, LLC / 2048 + 1), "");
 int main() { return 0; }
 ''')
-    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-loop-limit=10000000", "-D__HIP_PLATFORM_AMD__",
+    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-fconstexpr-loop-limit=10000000",
+                        "-fconstexpr-ops-limit=1000000000", "-D__HIP_PLATFORM_AMD__",
                         f"-I{ROOT / 'include'}", f"-I{ROOT / 'fufft_amd' / 'csrc'}", f"-I{rocm / 'include'}", str(src)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr

@@ -89,8 +89,10 @@ __global__ void __launch_bounds__(C * (H / V)) col_kernel(const ColParams p)
    const uint32_t dro = (uint32_t)(L * V) * W8 + c * 8u;     // row slot L*V, column c
 
    // whole lines are written through; the halves and quarters of narrower tiles
-   // are left to the L2 to put together (512 rows, 8 columns, 8 M points 73.5 ->
-   // 78.9 us written through)
+   // are left to the L2 to put together.  us, left / written through, 8 or 4 columns:
+   // conv 512 x 512, 8 M points 68.7 / 70.2, 4 M 37.9 / 37.9, real pairs 2.4 M 26.1 / 27.0;
+   // conv 2048 x 2048, 33 M 354 / 364; split apply 512 x 512, 2.4 M 17.3 / 18.3.  (Complex
+   // convs of 0.5 to 2.4 M points alone gain: 512 x 512, 1 M 16.5 / 14.1, 2.4 M 28.9 / 26.7.)
    constexpr int ST_POL = C == 16 ? POL_WT : POL_DEFAULT;
    float2* A = lds + col * SLOTC;
    Twiddles<PL> tw;

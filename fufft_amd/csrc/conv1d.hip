@@ -364,24 +364,26 @@ __device__ __forceinline__ void conv1d_body(const Conv1dParams& p, const uint32_
 // forward N = 4096 442 / 425 (33 M points 122 / 113); a filter per signal N = 2048
 // lane-major 519 / 512, digit order 514 / 502.  Some kinds are faster straight: the
 // split apply (a spectrum and a filter per transform, N = 1024 570 / 604; one
-// spectrum, N = 4096 373 / 387), the near conv (N = 1024, 8 M points 23.65 / 23.95),
-// the chain at N = 8192 (1 M 10.6 / 10.9), the four-step middle but for N = 512
-// (65536 points x 160 80.4 / 81.3, 262144 x 12 27.5 / 27.9, 2^20 x 3 with own filters
-// 30.1 / 30.6; N = 512 the other way, 131072 x 24 28.8 / 28.0), and a filter per signal
-// at N = 1024 lane-major (526 / 535) and N = 4096 digit order (4 M 18.4 / 19.0).
-template<int N, int KIND>
+// spectrum, N = 4096 373 / 387), the conv of N = 8192 at radix 8 (digit order 515 /
+// 520), the near conv (N = 1024, 8 M points 23.65 / 23.95), the chain at N = 8192 (1 M
+// 10.6 / 10.9), the four-step middle but for N = 512 (65536 points x 160 80.4 / 81.3,
+// 262144 x 12 27.5 / 27.9, 2^20 x 3 with own filters 30.1 / 30.6; N = 512 the other
+// way, 131072 x 24 28.8 / 28.0), and a filter per signal at N = 1024 lane-major (526 /
+// 535) and N = 4096 digit order (4 M 18.4 / 19.0).
+template<int N, int V, int KIND>
 constexpr bool conv_straight()
 {
    if(conv_loops<N, KIND>()) return false;
    return KIND == K_APPLY || KIND == K_CONV_NEAR || KIND == K_CONV_CHAIN || (KIND == K_CONV_MID && N > 512) ||
-          (KIND == K_CONV_PSF && N == 1024) || (KIND == K_CONV_PSF_DR && N == 4096);
+          (KIND == K_CONV && N == 8192 && V == 8) || (KIND == K_CONV_PSF && N == 1024) ||
+          (KIND == K_CONV_PSF_DR && N == 4096);
 }
 
 template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_straight<N, KIND>()) {
+   if constexpr(conv_straight<N, V, KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, false>(p, blockIdx.x);
    } else {
       const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
@@ -396,7 +398,7 @@ template<int N, int V, int LAYOUT, int KIND, int MID>
 __global__ void __launch_bounds__(cpb_for(N / V) * (N / V))
 conv1d_bperm_kernel(const Conv1dParams p)
 {
-   if constexpr(conv_straight<N, KIND>()) {
+   if constexpr(conv_straight<N, V, KIND>()) {
       conv1d_body<N, V, LAYOUT, KIND, MID, true>(p, blockIdx.x);
    } else {
       const uint32_t iters = conv_loops<N, KIND>() ? p.iters : 1u;
